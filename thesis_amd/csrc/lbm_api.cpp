@@ -39,6 +39,7 @@ struct lbm_ctx {
     uint32_t* nodew = nullptr;    // compact node words
     uint32_t* rowmeta = nullptr;  // per row and word: fluid mask, first compact index
     uint32_t* blk = nullptr;      // per workgroup: first row, rows spanned
+    uint32_t* edge = nullptr;     // compact indices of the nodes k_edge closes
     uint32_t* qslot = nullptr;    // curved walls: per compact node, row of qv
     double* qv = nullptr;         // curved walls: 19 wall fractions per row
     size_t nf = 0;                // non-solid nodes
@@ -329,6 +330,23 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
         }
         if (qv.empty()) qv.assign(19, 0.0);
     }
+    // Extrapolating outlets and curved walls of 3D lattices with faces: k_step
+    // leaves their closures out and k_edge takes these nodes after it, where
+    // what the smaller k_step saves is more than the second launch costs (6 us).
+    // TRT duct 2n x n x n with wet-node walls and an extrapolating outlet, one
+    // launch / two: FP64 n = 48 24.8 / 27.9 us, 64 49.2 / 43.8, 128 352 / 253;
+    // FP32 n = 64 26.1 / 30.1, 80 49.3 / 46.0, 128 164 / 148.  The line lies
+    // between, at 56 MiB of populations.
+    std::vector<uint32_t> edge;
+    const bool periodic3 = p->periodic[0] && p->periodic[1] && p->periodic[2];
+    if (p->q == 19 && !periodic3 && nf * 19 * storage_bytes(p->storage) >= (size_t)56 << 20) {
+        const bool ext = p->outlet_model == LBM_OUTLET_EXTRAP2 || p->outlet_model == LBM_OUTLET_EXTRAP1;
+        for (size_t j = 0; j < nf; ++j) {
+            const uint32_t nd = nodew[j], cls = nd >> kClsShift;
+            const bool outlet = ext && (cls == LBM_PRES_E || (cls >= LBM_OUT_W && cls <= LBM_OUT_T));
+            if (outlet || (p->wall_model == LBM_WALL_CURVED && (nd & kBBMask))) edge.push_back((uint32_t)j);
+        }
+    }
     // Row metadata of the rank step: per row and 32-node word, the fluid mask
     // and the compact index of the word's first fluid node; per 256-node
     // workgroup, its first row and the number of rows it spans.
@@ -479,6 +497,7 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
     if (st == LBM_OK) st = dalloc(c, (void**)&c->nodew, sizeof(uint32_t) * (nf > 0 ? nf : 1));
     if (st == LBM_OK) st = dalloc(c, (void**)&c->rowmeta, sizeof(uint32_t) * rowmeta.size());
     if (st == LBM_OK) st = dalloc(c, (void**)&c->blk, sizeof(uint32_t) * blk.size());
+    if (st == LBM_OK && !edge.empty()) st = dalloc(c, (void**)&c->edge, sizeof(uint32_t) * edge.size());
     if (st == LBM_OK && !qslot.empty()) {
         st = dalloc(c, (void**)&c->qslot, sizeof(uint32_t) * qslot.size());
         if (st == LBM_OK) st = dalloc(c, (void**)&c->qv, sizeof(double) * qv.size());
@@ -523,6 +542,8 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
         k.npt = (v == 2 || v == 4) && (int)rblock / v >= 64 ? v : 1;
     }
     k.simple = simple ? 1 : 0;
+    k.edge = c->edge;
+    k.nedge = (uint32_t)edge.size();
     k.qslot = c->qslot;
     k.qv = c->qv;
     // the rank step addresses the tile layout (SoA planes only in its 16-bit
@@ -540,6 +561,7 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
         (nf > 0 && h2d(c->nodew, nodew.data(), sizeof(uint32_t) * nf) != hipSuccess) ||
         h2d(c->rowmeta, rowmeta.data(), sizeof(uint32_t) * rowmeta.size()) != hipSuccess ||
         h2d(c->blk, blk.data(), sizeof(uint32_t) * blk.size()) != hipSuccess ||
+        (c->edge && h2d(c->edge, edge.data(), sizeof(uint32_t) * edge.size()) != hipSuccess) ||
         (c->qslot && h2d(c->qslot, qslot.data(), sizeof(uint32_t) * qslot.size()) != hipSuccess) ||
         (c->qv && h2d(c->qv, qv.data(), sizeof(double) * qv.size()) != hipSuccess))
         return cleanup(LBM_EDEVICE);
@@ -564,7 +586,7 @@ void lbm_destroy(lbm_ctx* c) {
     if (!c) return;
     if (c->stream) hipStreamSynchronize(c->stream);
     void* bufs[] = {c->Palloc[0], c->Palloc[1], c->node, c->cidx, c->didx, c->nodew, c->rowmeta, c->blk, c->rho, c->u, c->v, c->w, c->up, c->vp, c->wp,
-                    c->rp, c->qslot, c->qv, c->ubc, c->vbc, c->wbc, c->fout, c->f1, c->fprev, c->om[0], c->om[1], c->frz, c->partials, c->out4};
+                    c->rp, c->edge, c->qslot, c->qv, c->ubc, c->vbc, c->wbc, c->fout, c->f1, c->fprev, c->om[0], c->om[1], c->frz, c->partials, c->out4};
     for (void* b : bufs)
         if (b) hipFree(b);
     if (c->ev0) hipEventDestroy(c->ev0);

@@ -741,7 +741,9 @@ __device__ inline void mref_shift(T* h, int sign) {
     for (int i = 0; i < L::Q; ++i) h[i] += (T)sign * (T)mref_off<L>(i);
 }
 
-template <class L, int S, bool OPEN>
+// HH, CURVED: whether the lattice may have wet-node and curved walls (kernels
+// compiled for lattices without them leave their code out).
+template <class L, int S, bool OPEN, bool HH = true, bool CURVED = true>
 __device__ inline void inflow_state(const typename Io<L, S>::raw* __restrict__ src, const KParams& kp,
                                     const Fields& fl, const uint32_t* __restrict__ cidx, uint32_t own,
                                     uint32_t nd, int x, int y, int z, size_t idx, typename Io<L, S>::T* h) {
@@ -749,16 +751,16 @@ __device__ inline void inflow_state(const typename Io<L, S>::raw* __restrict__ s
     uint32_t cn[L::Q];
     source_index<L, OPEN>(cidx, kp, x, y, z, cn);
     gather<L, S, OPEN>(src, kp, own, nd, cn, h);
-    if (kp.wall == 3 && (nd & kBBMask)) bouzidi<L, S>(src, kp, own, nd, cn, h);
+    if (CURVED && kp.wall == 3 && (nd & kBBMask)) bouzidi<L, S>(src, kp, own, nd, cn, h);
     const uint32_t cls = nd >> kClsShift;
     if (OPEN && L::Q == 9 && cls == VEL_W) zou_inlet<L, T>(kp, fl, idx, nd, h);
     if (OPEN && L::Q == 9 && cls == VEL_N) zou_lid<L, T>(kp, fl, idx, nd, h);
     // velocity faces and wet-node walls mix link speeds: they act on f - w
-    const bool conv = L::Q == 19 && kp.mref && ((OPEN && cls != FLUID) || kp.wall == 2);
+    const bool conv = L::Q == 19 && kp.mref && ((OPEN && cls != FLUID) || (HH && kp.wall == 2));
     if (conv) mref_shift<L, T>(h, -1);
     if (OPEN && L::Q == 19) vel3d<L, T>(kp, fl, idx, cls, h);
     if (kp.wall == 1 && (nd & kBBMask)) onnode_walls<L, T>(nd, h);
-    if (L::Q == 19 && kp.wall == 2) hh_walls<L, T>(nd, h);
+    if (HH && L::Q == 19 && kp.wall == 2) hh_walls<L, T>(nd, h);
     if (conv) mref_shift<L, T>(h, 1);
 }
 
@@ -839,6 +841,48 @@ __device__ inline void extrap_mix(T* f, const T* ha, const T* hb, bool second) {
     for (int i = 0; i < L::Q; ++i)
         if (G * cmp<L>(i, A) > 0) f[i] = second ? (T)2 * ha[i] - hb[i] : ha[i];
 }
+// Term k of an extrapolating outlet node's populations: k = 0 its own (all of
+// them), then the unknowns from the nodes upstream, 2 f(x+n) - f(x+2n) (second)
+// or f(x+n).
+template <class L, class T, int A, int G>
+__device__ inline void extrap_put(int k, bool second, const T* hk, T* h) {
+#pragma unroll
+    for (int i = 0; i < L::Q; ++i)
+        if (G * cmp<L>(i, A) > 0) h[i] = k == 2 ? h[i] - hk[i] : second ? (T)2 * hk[i] : hk[i];
+}
+template <class L, class T>
+__device__ inline void extrap_term(uint32_t cls, int k, bool second, const T* hk, T* h) {
+    if (k == 0) {
+#pragma unroll
+        for (int i = 0; i < L::Q; ++i) h[i] = hk[i];
+        return;
+    }
+    switch (cls) {
+    case PRES_E: extrap_put<L, T, 0, -1>(k, second, hk, h); break;
+    case OUT_W: extrap_put<L, T, 0, 1>(k, second, hk, h); break;
+    case OUT_S: extrap_put<L, T, 1, 1>(k, second, hk, h); break;
+    case OUT_N: extrap_put<L, T, 1, -1>(k, second, hk, h); break;
+    case OUT_B: extrap_put<L, T, 2, 1>(k, second, hk, h); break;
+    default: extrap_put<L, T, 2, -1>(k, second, hk, h); break;
+    }
+}
+// The outlet models that need the node alone (pressure, f_eq); they act on
+// f - w (extrapolations, whose coefficients sum to one, do not need it).
+template <class L, int S, bool OPEN>
+__device__ inline void outlet3_local(const KParams& kp, const Fields& fl, size_t idx, uint32_t cls,
+                                     typename Io<L, S>::T* f) {
+    using T = typename Io<L, S>::T;
+    if (kp.mref) mref_shift<L, T>(f, -1);
+    switch (cls) {
+    case PRES_E: outlet3_face<L, S, OPEN, 0, -1>(kp, fl, idx, f); break;
+    case OUT_W: outlet3_face<L, S, OPEN, 0, 1>(kp, fl, idx, f); break;
+    case OUT_S: outlet3_face<L, S, OPEN, 1, 1>(kp, fl, idx, f); break;
+    case OUT_N: outlet3_face<L, S, OPEN, 1, -1>(kp, fl, idx, f); break;
+    case OUT_B: outlet3_face<L, S, OPEN, 2, 1>(kp, fl, idx, f); break;
+    default: outlet3_face<L, S, OPEN, 2, -1>(kp, fl, idx, f); break;
+    }
+    if (kp.mref) mref_shift<L, T>(f, 1);
+}
 template <class L, int S, bool OPEN>
 __device__ inline void outlet3d(const typename Io<L, S>::raw* __restrict__ src, const KParams& kp, const Fields& fl,
                                 const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ nodew, bool compact,
@@ -879,18 +923,7 @@ __device__ inline void outlet3d(const typename Io<L, S>::raw* __restrict__ src, 
         default: extrap_mix<L, T, 2, -1>(f, ha, hb, second); break;
         }
     } else {
-        // the pressure and f_eq closures act on f - w (extrapolations, whose
-        // coefficients sum to one, do not need it)
-        if (kp.mref) mref_shift<L, T>(f, -1);
-        switch (cls) {
-        case PRES_E: outlet3_face<L, S, OPEN, 0, -1>(kp, fl, idx, f); break;
-        case OUT_W: outlet3_face<L, S, OPEN, 0, 1>(kp, fl, idx, f); break;
-        case OUT_S: outlet3_face<L, S, OPEN, 1, 1>(kp, fl, idx, f); break;
-        case OUT_N: outlet3_face<L, S, OPEN, 1, -1>(kp, fl, idx, f); break;
-        case OUT_B: outlet3_face<L, S, OPEN, 2, 1>(kp, fl, idx, f); break;
-        default: outlet3_face<L, S, OPEN, 2, -1>(kp, fl, idx, f); break;
-        }
-        if (kp.mref) mref_shift<L, T>(f, 1);
+        outlet3_local<L, S, OPEN>(kp, fl, idx, cls, f);
     }
 #pragma unroll
     for (int i = 0; i < L::Q; ++i) h[i] = f[i];

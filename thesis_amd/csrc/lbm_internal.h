@@ -62,6 +62,8 @@ struct KParams {
     int rmax;                // rows staged per workgroup (LDS sizing)
     const uint2* rowmeta;    // per row and word: (fluid mask, compact index of first fluid node)
     const uint2* blk;        // per rblock-node workgroup: (first row, rows spanned)
+    const uint32_t* edge;    // compact indices of the nodes that k_edge closes after k_step (nedge 0: none)
+    uint32_t nedge;
     const uint32_t* qslot;   // curved walls: per compact node, its row of qv (0xFFFFFFFF: none)
     const double* qv;        // curved walls: 19 wall fractions per row
     // FP32 copies of omega, omega_m, g and g / 2 (set_float_params): float
@@ -95,6 +97,9 @@ struct Fields {              // FP64 side arrays (N each)
 hipError_t launch_step(int q, int storage, int collision, bool open, const KParams& kp,
                        const void* src, void* dst, const uint32_t* node, const uint32_t* cidx, Fields fl,
                        bool write_macros, hipStream_t st);
+// D3Q19: the kp.nedge nodes of kp.edge, after k_step of the same step.
+hipError_t launch_edge(int storage, int collision, const KParams& kp, const void* src, void* dst,
+                       const uint32_t* cidx, const Fields& fl, bool write_macros, hipStream_t st);
 hipError_t launch_recon(int q, int storage, bool open, const KParams& kp, const void* src,
                         const uint32_t* node, const uint32_t* cidx, Fields fl, hipStream_t st);
 hipError_t launch_init(int q, int storage, int collision, int mode, const KParams& kp, void* dst,
