@@ -69,6 +69,20 @@ __device__ inline void pull(const typename CIo<S>::raw* __restrict__ src, const 
         r[i] = CIo<S>::ld(src, (uint32_t)(19 + i) * cp.plane + k, i, true);
     }
 }
+// The FP64 two-launch step's pull: each plane the scalar base of its load and
+// one 32-bit byte offset per link for both colours (k_cg3_psi: 100 -> 62
+// registers); red(i, r_i) receives the red populations when R.
+template <bool R, class Red>
+__device__ inline void pull64(const double* __restrict__ src, const CgParams& cp, int x, int y, int z, double* h,
+                              Red red) {
+#pragma unroll
+    for (int i = 0; i < 19; ++i) {
+        const int sx = wrap(x - CX[i], cp.nx), sy = wrap(y - CY[i], cp.ny), sz = wrap(z - CZ[i], cp.nz);
+        const uint32_t k = (((uint32_t)sz * (uint32_t)cp.ny + (uint32_t)sy) * (uint32_t)cp.nx + (uint32_t)sx) * 8u;
+        h[i] = *(const double*)((const char*)(src + (uint32_t)i * cp.plane) + k);
+        if (R) red(i, *(const double*)((const char*)(src + (uint32_t)(19 + i) * cp.plane) + k));
+    }
+}
 
 template <class T>
 __device__ inline void densities(const T* h, const T* r, T& rho, T& rr) {
@@ -193,6 +207,46 @@ __device__ inline void gradient(const CgParams& cp, int x, int y, int z, Psi psi
     gx = ax; gy = ay; gz = az;
 }
 
+// gradient<H> of a field in the workgroup's LDS tile.
+//
+// The tile: the workgroup's 64 x 4 nodes of plane z with their H-node frame in
+// x, y and z of a field f (linear node index), about 11 loads per thread in
+// place of the 104 of the large stencil (5 of 18 with H = 1).
+template <int H, class T> struct Tile {
+    static constexpr int W = BX + 2 * H, R = BY + 2 * H, D = 2 * H + 1, N = W * R * D;
+    __device__ static void load(T* t, const T* __restrict__ f, const CgParams& cp, int x0, int y0, int z) {
+        for (int e = threadIdx.y * BX + threadIdx.x; e < N; e += BX * BY) {
+            const int pl = e / (W * R), r = e - pl * (W * R), ly = r / W, lx = r - ly * W;
+            const int gx = x0 - H + lx, gy = y0 - H + ly;
+            if (gx >= cp.nx + H || gy >= cp.ny + H) continue;   // beyond the box and its frame
+            t[e] = f[((uint32_t)wrap(z - H + pl, cp.nz) * (uint32_t)cp.ny + (uint32_t)wrap(gy, cp.ny)) *
+                         (uint32_t)cp.nx + (uint32_t)wrap(gx, cp.nx)];
+        }
+    }
+    __device__ static T get(const T* t, int dx, int dy, int dz) {
+        return t[((dz + H) * R + (int)threadIdx.y + dy + H) * W + (int)threadIdx.x + dx + H];
+    }
+};
+template <int H, class T>
+__device__ inline void gradient_tile(const T* t, T& gx, T& gy, T& gz) {
+    T ax = 0, ay = 0, az = 0;
+#pragma unroll
+    for (int dz = -H; dz <= H; ++dz)
+#pragma unroll
+        for (int dy = -H; dy <= H; ++dy)
+#pragma unroll
+            for (int dx = -H; dx <= H; ++dx) {
+                const int c2 = dx * dx + dy * dy + dz * dz;
+                const double wk = H == 1 ? LOW(c2) : HOW(c2);
+                if (wk == 0.0) continue;
+                const T p = (T)wk * Tile<H, T>::get(t, dx, dy, dz);
+                if (dx) ax += (T)dx * p;
+                if (dy) ay += (T)dy * p;
+                if (dz) az += (T)dz * p;
+            }
+    gx = ax; gy = ay; gz = az;
+}
+
 // The workgroup's (x, y, z) block from its dispatch order renumbered by
 // xcd_block, so that the row blocks an XCD runs together are neighbours in y
 // and share their neighbour rows' lines in that XCD's L2.
@@ -208,7 +262,10 @@ __device__ inline bool node_of(const CgParams& cp, int& x, int& y, int& z) {
 }
 
 // Phase field of the post-streaming state (and with E its density in the
-// second half of psi).
+// second N of psi).  FP64 storage keeps the red density too, in the third N: the
+// collision needs the red populations only through their sum, so the step then
+// pulls the deviations alone.  Not so in FP32 and FP16, where it measured no
+// gain (100 x 90 x 80: 71 us both ways).
 template <int S, bool E>
 __global__ __launch_bounds__(BX * BY) void k_cg3_psi(const typename CIo<S>::raw* __restrict__ src, CgParams cp,
                                                      typename CIo<S>::T* __restrict__ psi) {
@@ -216,13 +273,17 @@ __global__ __launch_bounds__(BX * BY) void k_cg3_psi(const typename CIo<S>::raw*
     int x, y, z;
     if (!node_of(cp, x, y, z)) return;
     T h[19], r[19], rho, rr;
-    pull<S>(src, cp, x, y, z, h, r);
+    if constexpr (S == 0) pull64<true>(src, cp, x, y, z, h, [&](int i, double v) { r[i] = v; });
+    else pull<S>(src, cp, x, y, z, h, r);
     densities<T>(h, r, rho, rr);
+    const size_t n = (size_t)cp.nx * cp.ny * cp.nz;
     const uint32_t j = ((uint32_t)z * (uint32_t)cp.ny + (uint32_t)y) * (uint32_t)cp.nx + (uint32_t)x;
     psi[j] = ((T)2 * rr - rho) / rho;
-    if (E) psi[(size_t)cp.nx * cp.ny * cp.nz + j] = rho;
+    if (E) psi[n + j] = rho;
+    if (S == 0) psi[2 * n + j] = rr;
 }
 
+// FP32 and FP16 storage (FP64: k_cg3_step64)
 template <int S, int H, bool E>
 __global__ __launch_bounds__(BX * BY) void k_cg3_step(const typename CIo<S>::raw* __restrict__ src,
                                                       typename CIo<S>::raw* __restrict__ dst,
@@ -251,6 +312,45 @@ __global__ __launch_bounds__(BX * BY) void k_cg3_step(const typename CIo<S>::raw
         const size_t n = (size_t)cp.nx * cp.ny * cp.nz;
         for (int a = 0; a < 6; ++a) mac[a * n + idx] = (double)m[a];
     }
+}
+
+// The FP64 step of the same: phase field (and density) from an LDS tile, red
+// density from k_cg3_psi.  128^3 per step, both launches: 18-point gradient
+// 369 -> 325 us, 104-point 464 -> 374 us (256 -> 188 registers), 64^3 enhanced
+// 104-point 150 -> 56 us (656 B of scratch -> none).
+template <int H, bool E>
+__global__ __launch_bounds__(BX * BY) void k_cg3_step64(const double* __restrict__ src, double* __restrict__ dst,
+                                                        const double* __restrict__ psi, CgParams cp,
+                                                        double* __restrict__ mac, int write_macros) {
+    using TL = Tile<H, double>;
+    __shared__ double lpsi[TL::N];
+    __shared__ double lrho[E ? TL::N : 1];
+    int x, y, z;
+    const bool in = node_of(cp, x, y, z);
+    const size_t n = (size_t)cp.nx * cp.ny * cp.nz;
+    TL::load(lpsi, psi, cp, x - (int)threadIdx.x, y - (int)threadIdx.y, z);
+    if (E) TL::load(lrho, psi + n, cp, x - (int)threadIdx.x, y - (int)threadIdx.y, z);
+    __syncthreads();
+    if (!in) return;
+    const uint32_t idx = ((uint32_t)z * (uint32_t)cp.ny + (uint32_t)y) * (uint32_t)cp.nx + (uint32_t)x;
+    // red populations that sum to the red density: x + (-0.0) is x
+    double h[19], r[19];
+    pull64<false>(src, cp, x, y, z, h, [](int, double) {});
+    r[0] = psi[2 * n + idx];
+#pragma unroll
+    for (int i = 1; i < 19; ++i) r[i] = -0.0;
+    double gx, gy, gz, d[3] = {0, 0, 0};
+    gradient_tile<H, double>(lpsi, gx, gy, gz);
+    if (E) gradient_tile<H, double>(lrho, d[0], d[1], d[2]);
+    double ho[19], ro[19], m[6];
+    collide<double, E>(cp, h, r, gx, gy, gz, d, ho, ro, m);
+#pragma unroll
+    for (int i = 0; i < 19; ++i) {
+        CIo<0>::st(dst, (uint32_t)i * cp.plane + idx, ho[i], i, false);
+        CIo<0>::st(dst, (uint32_t)(19 + i) * cp.plane + idx, ro[i], i, true);
+    }
+    if (write_macros)
+        for (int a = 0; a < 6; ++a) mac[a * n + idx] = m[a];
 }
 
 // Single-pass step for the 18-point gradient.  A workgroup owns a 64 x TY
@@ -446,6 +546,19 @@ __global__ __launch_bounds__(BX * BY) void k_cg3_recon(const typename CIo<S>::ra
     }
 }
 
+template <int S, int H, bool E>
+static void two_launches(dim3 grid, dim3 block, const void* src, void* dst, void* psi, const CgParams& cp, double* mac,
+                         int w, hipStream_t st) {
+    using R = typename CIo<S>::raw;
+    using T = typename CIo<S>::T;
+    hipLaunchKernelGGL((k_cg3_psi<S, E>), grid, block, 0, st, (const R*)src, cp, (T*)psi);
+    if constexpr (S == 0)
+        hipLaunchKernelGGL((k_cg3_step64<H, E>), grid, block, 0, st, (const R*)src, (R*)dst, (const T*)psi, cp, mac, w);
+    else
+        hipLaunchKernelGGL((k_cg3_step<S, H, E>), grid, block, 0, st, (const R*)src, (R*)dst, (const T*)psi, cp, mac,
+                           w);
+}
+
 inline dim3 grid_of(const CgParams& cp) { return dim3((cp.nx + BX - 1) / BX, (cp.ny + BY - 1) / BY, cp.nz); }
 
 }  // namespace cg3
@@ -475,14 +588,7 @@ hipError_t cg3_launch_step(int storage, int ho, const void* src, void* dst, void
 #undef CG3_FZT_
         return hipGetLastError();
     }
-#define CG3_STEP_(S_, H_, E_)                                                                                  \
-    do {                                                                                                       \
-        using R_ = typename cg3::CIo<S_>::raw;                                                                 \
-        using T_ = typename cg3::CIo<S_>::T;                                                                   \
-        hipLaunchKernelGGL((cg3::k_cg3_psi<S_, E_>), grid, block, 0, st, (const R_*)src, cp, (T_*)psi);        \
-        hipLaunchKernelGGL((cg3::k_cg3_step<S_, H_, E_>), grid, block, 0, st, (const R_*)src, (R_*)dst,        \
-                           (const T_*)psi, cp, mac, w);                                                        \
-    } while (0)
+#define CG3_STEP_(S_, H_, E_) cg3::two_launches<S_, H_, E_>(grid, block, src, dst, psi, cp, mac, w, st)
 #define CG3_STEP(S_, H_) do { if (cp.enhanced) CG3_STEP_(S_, H_, true); else CG3_STEP_(S_, H_, false); } while (0)
     if (storage == 0) { if (ho) CG3_STEP(0, 2); else CG3_STEP(0, 1); }
     else if (storage == 1) { if (ho) CG3_STEP(1, 2); else CG3_STEP(1, 1); }

@@ -28,7 +28,7 @@ struct lbm_cg_ctx {
     int64_t steps = -1;
     double* mac = nullptr;       // 6 N: rho_r, rho_b, rho, u, v, w
     double* rr0 = nullptr;       // 2 N initial densities
-    void* psi = nullptr;         // 2 N phase field and density (D3Q19)
+    void* psi = nullptr;         // 3 N phase field, density, red density (D3Q19)
     double* fout = nullptr;      // 2 q N: populations in and out
     double* partials = nullptr;
     bool walls = false;          // walls or body force: the reference-order path (lbm_cgw.hip)
@@ -51,6 +51,32 @@ lbm_status cfail(lbm_cg_ctx* c, lbm_status s, const char* fmt, ...) {
         hipError_t e_ = (expr);                                                            \
         if (e_ != hipSuccess) return cfail((c), LBM_EDEVICE, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
+// Column height of the single-pass D3Q19 step; 0: the two-launch step.
+//
+// Below 2^20 nodes, where the populations stay in the caches, two launches are
+// faster with FP64 and FP32 storage (FP32 per step: 64^3 21 / 23 us, 128 x 96 x 64
+// 59 / 68 us, 128 x 128 x 64 89 / 84 us); the two give the same bits there, not
+// with FP16, which keeps the single pass.
+//
+// One workgroup of 64 x 8 nodes
+// fits a CU (139-254 registers), and a column costs its planes and two more for
+// the phase field below and above, so the height is the one with the smallest
+// (rounds of 256 workgroups) x (planes + 2).  128^3 per step: 229 us with 128
+// columns of 32 planes, 156 us with 256 of 16 (FP16: 311 us with 64 columns of 64,
+// 95 us).  At most 32 planes (64 with FP16 storage): taller columns lose more
+// to the caches (256^3 FP32 1.153 ms at 32, 1.206 ms at 64).
+int cg3_zchunk(int nx, int ny, int nz, int rows, int storage) {
+    if (storage != LBM_STORE_F16 && (size_t)nx * ny * nz < (size_t)1 << 20) return 0;
+    const long tiles = (long)(nx / 64) * (ny / rows), cus = 256;
+    const int most = storage == LBM_STORE_F16 ? 64 : 32;
+    int best = most;
+    long cost = -1;
+    for (int zc = most; zc >= 1; --zc) {
+        const long rounds = (tiles * ((nz + zc - 1) / zc) + cus - 1) / cus, c = rounds * (zc + 2);
+        if (cost < 0 || c < cost) { cost = c; best = zc; }
+    }
+    return best;
+}
 size_t sbytes(int s) { return s == LBM_STORE_F64 ? 8 : s == LBM_STORE_F32 ? 4 : 2; }
 }  // namespace
 
@@ -95,17 +121,16 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
     k.xchunk_shift = 3;
     lbm::log2_env("LBM_XCD", k.xcd_shift);
     lbm::log2_env("LBM_XCHUNK", k.xchunk_shift);
-    // D3Q19 with the 18-point gradient on boxes of whole 64 x 8 row tiles:
-    // the single-pass step over z-columns of 32 planes (64 with FP16 storage:
-    // 0.756 vs 0.767 ms at 256^3; FP32 1.162 at 32, 1.220 at 64);
-    // LBM_CG3_ZCHUNK sets the column height (0 selects the two-launch step),
-    // LBM_CG3_ROWS the tile's rows (8 or 4)
+    // D3Q19 with the 18-point gradient on boxes of whole 64 x 8 row tiles: the
+    // single-pass step over z-columns of zchunk planes.  LBM_CG3_ZCHUNK sets the
+    // column height (0 selects the two-launch step), LBM_CG3_ROWS the tile's
+    // rows (8 or 4).
     k.zchunk = 0;
     k.zrows = 8;
     if (const char* e = std::getenv("LBM_CG3_ROWS"))
         if (std::strtol(e, nullptr, 10) == 4) k.zrows = 4;
     if (three_d && !p->high_order && p->nx % 64 == 0 && p->ny % k.zrows == 0) {
-        k.zchunk = p->storage == LBM_STORE_F16 ? 64 : 32;
+        k.zchunk = cg3_zchunk(p->nx, p->ny, nz, k.zrows, p->storage);
         if (const char* e = std::getenv("LBM_CG3_ZCHUNK")) {
             const long v = std::strtol(e, nullptr, 10);
             if (v >= 0 && v <= 4096) k.zchunk = (int)v;
@@ -124,7 +149,7 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
     ok = ok && hipMalloc(&c->P[0], pb) == hipSuccess && hipMalloc(&c->P[1], pb) == hipSuccess &&
          hipMalloc((void**)&c->mac, 6 * n * 8) == hipSuccess && hipMalloc((void**)&c->rr0, 2 * n * 8) == hipSuccess &&
          hipMalloc((void**)&c->partials, (size_t)kRedBlocks * lbm::cg::NRED * 8) == hipSuccess &&
-         (!three_d || hipMalloc(&c->psi, 2 * n * 8) == hipSuccess) &&
+         (!three_d || hipMalloc(&c->psi, 3 * n * 8) == hipSuccess) &&
          hipMemset(c->mac + 5 * n, 0, n * 8) == hipSuccess;
     if (!ok) {
         lbm_cg_destroy(c);
