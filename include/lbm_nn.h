@@ -39,6 +39,25 @@ int nn_col2im3x3(const float* dcol, int Bn, int H, int W, int C, int Kp, float* 
 int nn_grad_bf16(const float* dy, const float* y, int64_t n, int relu, void* dz, void* stream);
 int nn_colsum(const float* dy, const float* y, int relu, int M, int N, float* db, void* stream);
 int nn_to_bf16(const float* x, int64_t n, void* y, void* stream);
+/* Convolutions without a stored im2col matrix, for the network's layers (3x3 with
+ * cin, cout in {32, 64, 128}; 3x3 with cin 4, cout 32; 1x1 with cin 32, cout <= 32;
+ * other shapes return 3).  Input of the convolution: mode 0 x, mode 1 x at half
+ * the resolution upsampled x2, mode 2 x + skip.  w: bf16 [cout][kp] in im2col
+ * column order.  Same bits as nn_im2col3x3 + nn_gemm_bf16.  The bf16 operands of
+ * these entries start at 16-byte boundaries (else 3). */
+int nn_conv(const float* x, const float* skip, int mode, int Bn, int H, int W, int cin, int cout, int k, const void* w,
+            int kp, const float* bias, int relu, float* y, void* stream);
+/* input gradient of a 3x3 convolution from dz (bf16 [p][cout]) and wt of
+ * nn_weight_t; same bits as nn_gemm_bf16 + nn_col2im3x3 */
+int nn_conv_dx(const void* dz, int Bn, int H, int W, int cin, int cout, const void* wt, float* dx, void* stream);
+/* dw[n*kp + tap*cin + c] += sum over pixels of dz x (input as in nn_conv) */
+int nn_conv_dw(const float* x, const float* skip, int mode, const void* dz, int Bn, int H, int W, int cin, int cout,
+               int k, int kp, float* dw, void* stream);
+/* per layer i < nlayers (at most 16): wt[to[i] + (tap*cin + c)*cout + n] = w[from[i] + n*kp + tap*cin + c] */
+int nn_weight_t(const void* w, int nlayers, const int64_t* from, const int64_t* to, const int* cin, const int* cout,
+                const int* kp, void* wt, void* stream);
+/* nn_grad_bf16 and nn_colsum in one pass (N 32, 64 or 128) */
+int nn_grad_sum(const float* dy, const float* y, int64_t n, int relu, int N, void* dz, float* db, void* stream);
 /* 2x2 average pooling and nearest x2 upsampling with their adjoints */
 int nn_avgpool2(const float* x, int Bn, int H, int W, int C, float* y, void* stream);
 int nn_avgpool2_bwd(const float* dy, int Bn, int H, int W, int C, float* dx, void* stream);

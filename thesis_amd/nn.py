@@ -15,6 +15,7 @@ RELU, ATOMIC, TRANSC = 0x1, 0x2, 0x4
 EXPORTED = [
     "nn_gemm_bf16", "nn_im2col3x3", "nn_col2im3x3", "nn_grad_bf16", "nn_colsum", "nn_to_bf16", "nn_avgpool2",
     "nn_avgpool2_bwd", "nn_up2", "nn_up2_bwd", "nn_xint", "nn_ymix", "nn_axpy", "nn_add", "nn_fill", "nn_mse", "nn_adam",
+    "nn_conv", "nn_conv_dx", "nn_conv_dw", "nn_weight_t", "nn_grad_sum",
 ]
 
 _lib = None
@@ -44,6 +45,11 @@ def load():
         "nn_fill": [f32, i64, vp, vp],
         "nn_mse": [vp, vp, vp, vp, i64, i32, f32, vp, vp, vp],
         "nn_adam": [vp, vp, vp, vp, i64, f32, f32, f32, f32, i64, vp, i64, vp],
+        "nn_conv": [vp, vp, i32, i32, i32, i32, i32, i32, i32, vp, i32, vp, i32, vp, vp],
+        "nn_conv_dx": [vp, i32, i32, i32, i32, i32, vp, vp, vp],
+        "nn_conv_dw": [vp, vp, i32, vp, i32, i32, i32, i32, i32, i32, i32, vp, vp],
+        "nn_weight_t": [vp, i32, vp, vp, vp, vp, vp, vp, vp],
+        "nn_grad_sum": [vp, vp, i64, i32, i32, vp, vp, vp],
     }
     for name, args in sig.items():
         fn = getattr(lib, name)
@@ -69,6 +75,36 @@ def _check(rc, name):
 def gemm(M, N, R, A, lda, ta, B, ldb, tb, Cm, ldc, bias=None, flags=0, splits=1):
     _check(load().nn_gemm_bf16(M, N, R, _p(A), lda, int(ta), _p(B), ldb, int(tb), _p(Cm), ldc, _p(bias), flags,
                                splits, _stream()), "nn_gemm_bf16")
+
+
+# input of a convolution: x, x upsampled x2, x + skip
+IN_X, IN_UP, IN_ADD = 0, 1, 2
+
+
+def conv(x, skip, mode, Bn, H, W, cin, cout, k, w, kp, bias, relu, y):
+    _check(load().nn_conv(_p(x), _p(skip), mode, Bn, H, W, cin, cout, k, _p(w), kp, _p(bias), int(relu), _p(y),
+                          _stream()), "nn_conv")
+
+
+def conv_dx(dz, Bn, H, W, cin, cout, wt, dx):
+    _check(load().nn_conv_dx(_p(dz), Bn, H, W, cin, cout, _p(wt), _p(dx), _stream()), "nn_conv_dx")
+
+
+def conv_dw(x, skip, mode, dz, Bn, H, W, cin, cout, k, kp, dw):
+    _check(load().nn_conv_dw(_p(x), _p(skip), mode, _p(dz), Bn, H, W, cin, cout, k, kp, _p(dw), _stream()),
+           "nn_conv_dw")
+
+
+def weight_t(w, layers, wt):
+    """layers: (from, to, cin, cout, kp) of each (at most 16)."""
+    n = len(layers)
+    f, t = ((i64 * n)(*[v[k] for v in layers]) for k in (0, 1))
+    ci, co, kp = ((i32 * n)(*[v[k] for v in layers]) for k in (2, 3, 4))
+    _check(load().nn_weight_t(_p(w), n, f, t, ci, co, kp, _p(wt), _stream()), "nn_weight_t")
+
+
+def grad_sum(dy, y, relu, N, dz, db):
+    _check(load().nn_grad_sum(_p(dy), _p(y), dy.numel(), int(relu), N, _p(dz), _p(db), _stream()), "nn_grad_sum")
 
 
 def im2col(x, Bn, H, W, Cc, Kp, col):

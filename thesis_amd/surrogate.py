@@ -141,53 +141,50 @@ class Net:
         self.t = 0
 
     # -- layers -----------------------------------------------------------
-    def _conv(self, x, Bn, H, W, li, cache):
+    def _conv(self, x, Bn, H, W, li, cache, mode=nn.IN_X, skip=None):
+        """Layer li on x (mode IN_UP: x at half the resolution, upsampled;
+        IN_ADD: x + skip); the backward pass reads x and skip again."""
         _, cin, cout, k, relu = ARCH[li]
         kp = kpad(cin, k)
-        M = Bn * H * W
-        col = torch.empty(M * kp, dtype=torch.int16, device=self.dev)
-        if k == 3:
-            nn.im2col(x, Bn, H, W, cin, kp, col)
-        else:
-            assert kp == cin
-            nn.to_bf16(x, col)
-        y = torch.empty(M * cout, dtype=torch.float32, device=self.dev)
+        y = torch.empty(Bn * H * W * cout, dtype=torch.float32, device=self.dev)
         wo, bo = self.wo[li], self.bo[li]
-        nn.gemm(M, cout, kp, col, kp, 0, self.wbf[wo:wo + cout * kp], kp, 0, y, cout,
-                self.w[bo:bo + cout], nn.RELU if relu else 0, 1)
-        cache[li] = (col, y, Bn, H, W)
+        nn.conv(x, skip, mode, Bn, H, W, cin, cout, k, self.wbf[wo:wo + cout * kp], kp, self.w[bo:bo + cout], relu, y)
+        cache[li] = (x, skip, mode, y, Bn, H, W)
         return y
 
     def _conv_bwd(self, dy, li, cache, need_dx=True):
         _, cin, cout, k, relu = ARCH[li]
         kp = kpad(cin, k)
-        col, y, Bn, H, W = cache[li]
+        x, skip, mode, y, Bn, H, W = cache[li]
         M = Bn * H * W
         wo, bo = self.wo[li], self.bo[li]
         dz = torch.empty(M * cout, dtype=torch.int16, device=self.dev)
-        nn.grad_bf16(dy, y, relu, dz)
-        nn.colsum(dy, y, relu, M, cout, self.g[bo:bo + cout])
-        bm = 256 if cout <= 32 else 128
-        tiles = -(-kp // bm) * -(-cout // (32 if cout <= 32 else 64 if cout <= 64 else 128))
-        splits = max(1, min(2048 // max(tiles, 1), M // 2048))
-        nn.gemm(kp, cout, M, col, kp, 1, dz, cout, 1, self.g[wo:wo + cout * kp], kp, None,
-                nn.ATOMIC | nn.TRANSC, splits)
+        if cout % 32 == 0:
+            nn.grad_sum(dy, y, relu, cout, dz, self.g[bo:bo + cout])
+        else:
+            nn.grad_bf16(dy, y, relu, dz)
+            nn.colsum(dy, y, relu, M, cout, self.g[bo:bo + cout])
+        nn.conv_dw(x, skip, mode, dz, Bn, H, W, cin, cout, k, kp, self.g[wo:wo + cout * kp])
         if not need_dx:
             return None
-        dcol = torch.empty(M * kp, dtype=torch.float32, device=self.dev)
-        nn.gemm(M, kp, cout, dz, cout, 0, self.wbf[wo:wo + cout * kp], kp, 1, dcol, kp, None, 0, 1)
         if k == 1:
-            return dcol
+            dx = torch.empty(M * kp, dtype=torch.float32, device=self.dev)
+            nn.gemm(M, kp, cout, dz, cout, 0, self.wbf[wo:wo + cout * kp], kp, 1, dx, kp, None, 0, 1)
+            return dx
         dx = torch.empty(M * cin, dtype=torch.float32, device=self.dev)
-        nn.col2im(dcol, Bn, H, W, cin, kp, dx)
+        wt, at = cache["wt"]
+        nn.conv_dx(dz, Bn, H, W, cin, cout, wt[at[li]:at[li] + 9 * cin * cout], dx)
         return dx
 
     def _new(self, n):
         return torch.empty(n, dtype=torch.float32, device=self.dev)
 
     # -- network ----------------------------------------------------------
-    def forward(self, x, Bn, H, W):
-        """x: FP32 device tensor (Bn*H*W*3) NHWC; returns (out, cache)."""
+    def forward(self, x, Bn, H, W, keep_input=True):
+        """x: FP32 device tensor (Bn*H*W*4) NHWC; returns (out, cache).  The
+        backward pass reads the input again: keep_input copies it, so that the
+        caller may overwrite x before then."""
+        x = x.clone() if keep_input else x
         c = {}
         I = INDEX
         a = self._conv(x, Bn, H, W, I["e1a"], c)
@@ -211,27 +208,13 @@ class Net:
         ym = self._new(a.numel())
         nn.ymix(xi, Bn, H4, W4, 128, ym)
         a = self._conv(ym, Bn, H4, W4, I["b2"], c)
-        u = self._new(Bn * H3 * W3 * 128)
-        nn.up2(a, Bn, H4, W4, 128, u)
-        a = self._conv(u, Bn, H3, W3, I["d3a"], c)
-        t = self._new(a.numel())
-        nn.add(a, s3, t)        # the convolution output stays intact for its ReLU mask
-        a = t
-        a = self._conv(a, Bn, H3, W3, I["d3b"], c)
-        u = self._new(Bn * H2 * W2 * 128)
-        nn.up2(a, Bn, H3, W3, 128, u)
-        a = self._conv(u, Bn, H2, W2, I["d2a"], c)
-        t = self._new(a.numel())
-        nn.add(a, s2, t)        # the convolution output stays intact for its ReLU mask
-        a = t
-        a = self._conv(a, Bn, H2, W2, I["d2b"], c)
-        u = self._new(Bn * H * W * 64)
-        nn.up2(a, Bn, H2, W2, 64, u)
-        a = self._conv(u, Bn, H, W, I["d1a"], c)
-        t = self._new(a.numel())
-        nn.add(a, s1, t)        # the convolution output stays intact for its ReLU mask
-        a = t
-        a = self._conv(a, Bn, H, W, I["d1b"], c)
+        # upsampling and skip sums happen where the next convolution reads them
+        a = self._conv(a, Bn, H3, W3, I["d3a"], c, nn.IN_UP)
+        a = self._conv(a, Bn, H3, W3, I["d3b"], c, nn.IN_ADD, s3)
+        a = self._conv(a, Bn, H2, W2, I["d2a"], c, nn.IN_UP)
+        a = self._conv(a, Bn, H2, W2, I["d2b"], c, nn.IN_ADD, s2)
+        a = self._conv(a, Bn, H, W, I["d1a"], c, nn.IN_UP)
+        a = self._conv(a, Bn, H, W, I["d1b"], c, nn.IN_ADD, s1)
         out = self._conv(a, Bn, H, W, I["out"], c)
         c["dims"] = (Bn, H, W)
         return out, c
@@ -242,6 +225,16 @@ class Net:
         I = INDEX
         Bn, H, W = c["dims"]
         H2, W2, H3, W3, H4, W4 = H // 2, W // 2, H // 4, W // 4, H // 8, W // 8
+        # transposed weights of the 3x3 layers whose input gradient is taken
+        at, layers, off = {}, [], 0
+        for li, (name, cin, cout, k, _) in enumerate(ARCH):
+            if k == 3 and name != "e1a":
+                at[li] = off
+                layers.append((self.wo[li], off, cin, cout, kpad(cin, k)))
+                off += 9 * cin * cout
+        wt = torch.empty(off, dtype=torch.int16, device=self.dev)
+        nn.weight_t(self.wbf, layers, wt)
+        c["wt"] = (wt, at)
         d = self._conv_bwd(dout, I["out"], c)
         d = self._conv_bwd(d, I["d1b"], c)            # gradient of relu(d1a) + s1
         ds1 = d
@@ -291,7 +284,7 @@ class Net:
 
     def step(self, x, target, mask, Bn, H, W, lr, wch):
         nn.fill(0.0, self.g)
-        out, c = self.forward(x, Bn, H, W)
+        out, c = self.forward(x, Bn, H, W, keep_input=False)
         loss, grad = self.loss_grad(out, target, mask, wch)
         self.backward(grad, c)
         self.t += 1
@@ -299,7 +292,7 @@ class Net:
         return loss
 
     def predict(self, X, Bn, H, W):
-        out, _ = self.forward(X, Bn, H, W)
+        out, _ = self.forward(X, Bn, H, W, keep_input=False)
         return out
 
     # -- persistence --------------------------------------------------------
