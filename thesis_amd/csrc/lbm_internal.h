@@ -100,6 +100,11 @@ hipError_t launch_step(int q, int storage, int collision, bool open, const KPara
 // D3Q19: the kp.nedge nodes of kp.edge, after k_step of the same step.
 hipError_t launch_edge(int storage, int collision, const KParams& kp, const void* src, void* dst,
                        const uint32_t* cidx, const Fields& fl, bool write_macros, hipStream_t st);
+// D2Q9, FP64 or FP32: `steps` steps in one launch over squares of 32 x 32 nodes
+// with a frame of halo >= steps recomputed nodes (tile layout, node-local faces).
+hipError_t launch_multi2(int storage, int collision, const KParams& kp, const void* src, void* dst,
+                         const uint32_t* node, const uint32_t* cidx, const Fields& fl, int steps, int halo,
+                         hipStream_t st);
 hipError_t launch_recon(int q, int storage, bool open, const KParams& kp, const void* src,
                         const uint32_t* node, const uint32_t* cidx, Fields fl, hipStream_t st);
 hipError_t launch_init(int q, int storage, int collision, int mode, const KParams& kp, void* dst,
