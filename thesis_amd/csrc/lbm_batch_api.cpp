@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstdarg>
@@ -31,6 +32,7 @@ struct lbm_batch {
     std::vector<int> par;           // host copy of the buffer holding each instance's newest state
     size_t ndense = 0, nslots = 0, nfluid = 0, maxn = 0;
     int ntiles = 0, grid = 0;
+    int halo = 1, nsquares = 0;   // several-step phases: steps a barrier, squares of all instances
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<void*> allocs;
@@ -168,7 +170,7 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
         B.pbase = (uint32_t)pbase;
         B.dbase = (uint32_t)dbase;
         B.tbase = (uint32_t)tbase;
-        B.pad = 0;
+        B.mtx = B.mbase = B.pad = 0;
         magic((uint32_t)I.nx, B.mx, B.sx);
         B.omega = I.omega;
         const double lam = I.trt_magic > 0 ? I.trt_magic : 3.0 / 16.0;
@@ -186,6 +188,33 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
         maxn = nn > maxn ? nn : maxn;
         if (dbase >= 0xFFFFFFFFull || pbase >= 0xFFFFFFFFull || tbase >= (size_t)INT_MAX)
             return reject("batch too large");
+    }
+    // Steps a barrier between checks: a phase of t steps costs about 25 us for the
+    // barrier (0.1 us a workgroup) and 6 + 1.25 t us for each round of 248 squares
+    // of 32 - 2t nodes a side; the t with the least time a step (lbm_api.cpp has the
+    // same model for one lattice).
+    auto squares = [&](int t) {
+        const int side = 32 - 2 * t;
+        size_t s = 0;
+        for (const BInst& B : hinst) s += (size_t)((B.nx + side - 1) / side) * ((B.ny + side - 1) / side);
+        return s;
+    };
+    int halo = 1;
+    double cost = 0;
+    for (int t = 2; t <= 10; ++t) {
+        const double c = (25.0 + std::ceil((double)squares(t) / 248.0) * (6.0 + 1.25 * t)) / t;
+        if (halo == 1 || c < cost) { cost = c; halo = t; }
+    }
+    const size_t nsq = squares(halo);
+    if (nsq >= (size_t)INT_MAX) return reject("batch too large");
+    {
+        size_t at = 0;
+        const int side = 32 - 2 * halo;
+        for (BInst& B : hinst) {
+            B.mbase = (uint32_t)at;
+            B.mtx = (uint32_t)((B.nx + side - 1) / side);
+            at += (size_t)B.mtx * ((B.ny + side - 1) / side);
+        }
     }
     const size_t raw = storage == LBM_STORE_F64 ? 8 : 4;
 
@@ -210,6 +239,8 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
     b->nfluid = nfluid;
     b->maxn = maxn;
     b->ntiles = (int)tbase;
+    b->halo = halo;
+    b->nsquares = (int)nsq;
     auto bad = [&](lbm_status s) {
         g_create_err = b->err;
         lbm_batch_destroy(b);
@@ -224,7 +255,8 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
     // workgroup per XCD of headroom below the occupancy query's co-residency,
     // so that a CU the runtime keeps back cannot leave the grid waiting
     const int head = maxb >= 64 ? 8 : (maxb > 1 ? 1 : 0);
-    b->grid = b->ntiles < maxb - head ? b->ntiles : maxb - head;
+    const int most = std::max(b->ntiles, b->nsquares);
+    b->grid = most < maxb - head ? most : maxb - head;
     if (hipStreamCreate(&b->stream) != hipSuccess || hipEventCreate(&b->ev0) != hipSuccess ||
         hipEventCreate(&b->ev1) != hipSuccess) {
         b->err = "stream or event creation failed";
@@ -319,7 +351,7 @@ lbm_status lbm_batch_run(lbm_batch* b, double tol, int32_t check_every, int64_t 
     if (max_steps > 0)
         BCHK(b, batch_run(b->storage == LBM_STORE_F64 ? 0 : 1, b->collision, b->inst, n, b->ntiles, b->P[0],
                           b->P[1], b->nodew, bfields(b), b->up, b->vp, b->bs, tol, check_every, (int)max_steps,
-                          b->grid, b->stream));
+                          b->halo, b->nsquares, b->grid, b->stream));
     BCHK(b, hipEventRecord(b->ev1, b->stream));
     std::vector<int> done(n);
     std::vector<double> res(n);

@@ -13,8 +13,10 @@ struct BInst {
     uint32_t pbase;       // first population slot of the instance (a multiple of 64)
     uint32_t dbase;       // first index in the concatenated per-node arrays
     uint32_t tbase;       // first kBatchTile-node tile of the instance in the tile numbering
-    uint32_t sx, pad;     // invariant-divisor shift and multiplier for nx
+    uint32_t sx;          // invariant-divisor shift and multiplier for nx
+    uint32_t mtx;         // squares per row of the several-step phases (lbm_square.h)
     uint64_t mx;
+    uint32_t mbase, pad;  // first square of the instance in the square numbering
     double omega, omega_m, rho_out;
 };
 
@@ -36,7 +38,7 @@ size_t batch_lds_bytes(int ninst);
 int batch_max_blocks(int storage, int collision, int ninst);
 hipError_t batch_run(int storage, int collision, const BInst* inst, int ninst, int ntiles, void* P0, void* P1,
                      const uint32_t* nodew, Fields fl, double* uprev, double* vprev, BState bs, double tol,
-                     int check_every, int max_steps, int grid_blocks, hipStream_t st);
+                     int check_every, int max_steps, int halo, int nsquares, int grid_blocks, hipStream_t st);
 hipError_t batch_init(int storage, int collision, const BInst* inst, int ninst, int ntiles, void* P,
                       const uint32_t* nodew, Fields fl, int only, hipStream_t st);
 hipError_t batch_recon(int storage, const BInst* inst, int i, uint32_t n, const void* P, const uint32_t* nodew,

@@ -15,24 +15,22 @@
 // 8.0 / 3.7, 78 / 33.  What bounds it: on few squares the launch and the chain of
 // LDS round trips (about 1.3 us a step FP64), on many the instructions of the node
 // update, 1.8 times with the frame of 4.
-#include "lbm_device.h"
+#include "lbm_square.h"
 
 namespace lbm {
-
-constexpr int kSide = 32, kNodes = kSide * kSide;
 
 // FULL: more squares than CUs; FP32 then keeps to 64 registers so that two
 // workgroups share a CU (4096 x 1024: 52.7 -> 33.1 us per step; with one square a
 // CU the tighter code only costs, 256 x 64 1.47 -> 1.57 us).
 template <int S, int C, bool FULL>
-__global__ __launch_bounds__(kNodes, S == 1 && FULL ? 8 : 4) void k_multi2(const typename Io<D2Q9, S>::raw* __restrict__ src,
+__global__ __launch_bounds__(kSquare, S == 1 && FULL ? 8 : 4) void k_multi2(const typename Io<D2Q9, S>::raw* __restrict__ src,
                                                    typename Io<D2Q9, S>::raw* __restrict__ dst,
                                                    const uint32_t* __restrict__ node,
                                                    const uint32_t* __restrict__ cidx, KParams kp, Fields fl, int steps,
                                                    int halo, uint32_t tx) {
     using L = D2Q9;
     using T = typename Io<L, S>::T;
-    __shared__ T lds[8][kNodes];   // populations 1..8; the rest population stays with its thread
+    __shared__ T lds[8][kSquare];
     const int tid = threadIdx.x, lx = tid & (kSide - 1), ly = tid / kSide;
     const int in = kSide - 2 * halo, nx = kp.nx, ny = kp.ny;
     const uint32_t b = xcd_block(blockIdx.x, gridDim.x, kp.xcd_shift, kp.xchunk_shift), by = b / tx;
@@ -48,65 +46,18 @@ __global__ __launch_bounds__(kNodes, S == 1 && FULL ? 8 : 4) void k_multi2(const
         nd = node[idx];
     }
     const bool live = own != kNone;
-    const uint32_t cls = nd >> kClsShift;
     T p[L::Q];   // the node's post-collision populations
 #pragma unroll
     for (int i = 0; i < L::Q; ++i) p[i] = live ? Io<L, S>::ld(src, tslot<L>(i, own), i) : (T)0;
-    // directions whose source is beyond a wall, and beyond a non-periodic face
-    uint32_t wall = 0, out = 0;
-    const bool xl = !kp.per[0] && x == 0, xh = !kp.per[0] && x == nx - 1;
-    const bool yl = !kp.per[1] && y == 0, yh = !kp.per[1] && y == ny - 1;
-#pragma unroll
-    for (int i = 1; i < L::Q; ++i) {
-        if ((nd >> L::opp(i)) & 1u) wall |= 1u << i;
-        else if ((L::cx(i) > 0 && xl) || (L::cx(i) < 0 && xh) || (L::cy(i) > 0 && yl) || (L::cy(i) < 0 && yh))
-            out |= 1u << i;
-    }
-    const bool half = kp.wall == 0;
-    const uint32_t links = __any((wall | out) != 0);   // uniform: whether any node of the wave has such a link
-    // the face's prescribed velocity, read once
-    double ub[2] = {0.0, 0.0};
+    const uint2 ln = square_links(nd, !kp.per[0] && x == 0, !kp.per[0] && x == nx - 1, !kp.per[1] && y == 0,
+                                  !kp.per[1] && y == ny - 1);
+    double ub[2] = {0.0, 0.0};   // the face velocity, read once
+    if (live && (nd >> kClsShift) != FLUID && fl.ubc) { ub[0] = fl.ubc[idx]; ub[1] = fl.vbc[idx]; }
     Fields fn = fl;
-    if (live && cls != FLUID && fl.ubc) { ub[0] = fl.ubc[idx]; ub[1] = fl.vbc[idx]; }
     fn.ubc = ub;
     fn.vbc = ub + 1;
+    square_steps<T, C>(kp, fn, idx, live, nd, ln.x, ln.y, steps, lds, p);
     const int rim = min(min(lx, kSide - 1 - lx), min(ly, kSide - 1 - ly));
-#pragma unroll
-    for (int i = 1; i < L::Q; ++i) lds[i - 1][tid] = p[i];
-    for (int s = 1; s <= steps; ++s) {
-        const bool on = live && rim >= s;
-        T h[L::Q];
-        __syncthreads();
-        if (on) {
-            h[0] = p[0];
-#pragma unroll
-            for (int i = 1; i < L::Q; ++i) {
-                h[i] = lds[i - 1][tid - L::cx(i) - kSide * L::cy(i)];
-            }
-            if (links) {
-#pragma unroll
-                for (int i = 1; i < L::Q; ++i) {
-                    const T w = half ? p[L::opp(i)] : p[i];
-                    h[i] = (wall >> i) & 1u ? w : ((out >> i) & 1u ? p[i] : h[i]);
-                }
-            }
-        }
-        __syncthreads();
-        if (on) {
-            if (cls != FLUID || links) {
-                if (cls == VEL_W) zou_inlet<L, T>(kp, fn, 0, nd, h);
-                if (cls == VEL_N) zou_lid<L, T>(kp, fn, 0, nd, h);
-                if (kp.wall == 1 && (nd & kBBMask)) onnode_walls<L, T>(nd, h);
-                if (cls == PRES_E) zou_outlet<L, T>(kp, fn, 0, h);
-            }
-            T drho, rho, u[3];
-            moments<L, T>(kp, cls, h, drho, rho, u);
-            frozen_macros<T>(kp, fl, cls, idx, drho, rho, u);
-            collide<L, T, C>(kp, h, drho, rho, u, p);
-#pragma unroll
-            for (int i = 1; i < L::Q; ++i) lds[i - 1][tid] = p[i];
-        }
-    }
     if (live && rim >= halo && ux < nx && uy < ny) {   // ux, uy >= 0 inside the frame
 #pragma unroll
         for (int i = 0; i < L::Q; ++i) sto(dst, tslot<L>(i, own), Io<L, S>::pk(p[i], i));
@@ -120,7 +71,7 @@ static hipError_t multi_t(const KParams& kp, const void* src, void* dst, const u
     const int in = kSide - 2 * halo;
     const uint32_t tx = (uint32_t)(kp.nx + in - 1) / in, ty = (uint32_t)(kp.ny + in - 1) / in;
     auto go = [&](auto k) {
-        hipLaunchKernelGGL(k, dim3(tx * ty), dim3(kNodes), 0, st, (const raw*)src, (raw*)dst, node, cidx, kp, fl, steps,
+        hipLaunchKernelGGL(k, dim3(tx * ty), dim3(kSquare), 0, st, (const raw*)src, (raw*)dst, node, cidx, kp, fl, steps,
                            halo, tx);
     };
     if (S == 1 && tx * ty > 256) go(k_multi2<S, C, true>);
