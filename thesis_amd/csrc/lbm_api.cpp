@@ -5,6 +5,7 @@
 // HIP stream and all device buffers; the loop enqueues one fused kernel per
 // step and synchronises the host once per call, not once per phase.
 #include "lbm.h"
+#include "lbm_hostcopy.h"
 #include "lbm_internal.h"
 
 #include <hip/hip_runtime.h>
@@ -442,6 +443,7 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
         delete c;
         return reject("no current HIP device");
     }
+    host_staging_retain();
     c->p = *p;
     c->p.nz = nz;
     c->q = p->q;
@@ -456,7 +458,7 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
     k.qstride = plane_stride(nf > 0 ? nf : 1, c->raw_bytes);
     k.qstride32 = (uint32_t)k.qstride;
     if (k.qstride * c->q * c->raw_bytes >= (1ull << 32) || n * 4 >= (1ull << 32)) {
-        delete c;
+        lbm_destroy(c);
         return reject("population buffer or node map above 4 GiB (32-bit offsets)");
     }
     k.nf = (uint32_t)nf;
@@ -630,6 +632,7 @@ void lbm_destroy(lbm_ctx* c) {
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
     if (c->stream) hipStreamDestroy(c->stream);
+    host_staging_release();
     delete c;
 }
 
@@ -799,9 +802,11 @@ lbm_status lbm_get_macros(lbm_ctx* c, double* rho, double* u, double* v, double*
     const size_t b = 8 * c->n;
     const double* srcs[4] = {c->rho, c->u, c->v, c->w};
     double* dsts[4] = {rho, u, v, w};
+    OutCopy out[4];
+    int n = 0;
     for (int a = 0; a < 4; ++a)
-        if (dsts[a]) HIPCHK(c, hipMemcpyAsync(dsts[a], srcs[a], b, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (dsts[a]) out[n++] = {dsts[a], srcs[a], b};
+    HIPCHK(c, copy_to_host(out, n, c->dev, c->stream));
     return LBM_OK;
 }
 
@@ -813,8 +818,8 @@ lbm_status lbm_get_f(lbm_ctx* c, double* f) {
     Fields fl = fields(c);
     if (c->om[0]) fl.om_in = c->om[(c->steps - 1) & 1];
     HIPCHK(c, launch_recon(c->q, c->p.storage, c->open, c->kp, c->P[c->cur ^ 1], c->node, c->cidx, fl, c->stream));
-    HIPCHK(c, hipMemcpyAsync(f, c->fout, 8 * c->n * c->q, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const OutCopy out = {f, c->fout, 8 * c->n * c->q};
+    HIPCHK(c, copy_to_host(&out, 1, c->dev, c->stream));
     return LBM_OK;
 }
 

@@ -8,6 +8,7 @@
 // (S/Iterate.cu:23-625).
 #include "lbm.h"
 #include "lbm_batch_internal.h"
+#include "lbm_hostcopy.h"
 
 #include <hip/hip_runtime.h>
 
@@ -32,6 +33,7 @@ struct lbm_batch {
     std::vector<int> par;           // host copy of the buffer holding each instance's newest state
     size_t ndense = 0, nslots = 0, nfluid = 0, maxn = 0;
     int ntiles = 0, grid = 0;
+    int dev = 0;                  // device current at creation
     int halo = 1, nsquares = 0;   // several-step phases: steps a barrier, squares of all instances
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -226,6 +228,8 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
         return reject("device does not support cooperative launches");
 
     lbm_batch* b = new lbm_batch();
+    host_staging_retain();
+    b->dev = dev;
     b->n = n;
     b->collision = collision;
     b->storage = storage;
@@ -295,6 +299,7 @@ void lbm_batch_destroy(lbm_batch* b) {
     if (b->ev0) hipEventDestroy(b->ev0);
     if (b->ev1) hipEventDestroy(b->ev1);
     if (b->stream) hipStreamDestroy(b->stream);
+    host_staging_release();
     delete b;
 }
 
@@ -380,9 +385,11 @@ lbm_status lbm_batch_get_macros(lbm_batch* b, int32_t i, double* rho, double* u,
     const size_t nn = (size_t)B.nx * B.ny, o = B.dbase;
     const double* src[3] = {b->rho + o, b->u + o, b->v + o};
     double* dst[3] = {rho, u, v};
+    OutCopy out[3];
+    int k = 0;
     for (int a = 0; a < 3; ++a)
-        if (dst[a]) BCHK(b, hipMemcpyAsync(dst[a], src[a], 8 * nn, hipMemcpyDeviceToHost, b->stream));
-    BCHK(b, hipStreamSynchronize(b->stream));
+        if (dst[a]) out[k++] = {dst[a], src[a], 8 * nn};
+    BCHK(b, copy_to_host(out, k, b->dev, b->stream));
     return LBM_OK;
 }
 
@@ -398,8 +405,8 @@ lbm_status lbm_batch_get_f(lbm_batch* b, int32_t i, double* f) {
     BCHK(b, hipMemsetAsync(b->fout, 0, 8 * 9 * nn, b->stream));
     BCHK(b, batch_recon(b->storage == LBM_STORE_F64 ? 0 : 1, b->inst, i, B.n, b->P[src], b->nodew, bfields(b),
                         b->fout, b->stream));
-    BCHK(b, hipMemcpyAsync(f, b->fout, 8 * 9 * nn, hipMemcpyDeviceToHost, b->stream));
-    BCHK(b, hipStreamSynchronize(b->stream));
+    const OutCopy out = {f, b->fout, 8 * 9 * nn};
+    BCHK(b, copy_to_host(&out, 1, b->dev, b->stream));
     return LBM_OK;
 }
 

@@ -1,6 +1,7 @@
 // C ABI of the colour-gradient step, D2Q9 and D3Q19 (declared in include/lbm.h).
 #include "lbm.h"
 #include "lbm_cg.h"
+#include "lbm_hostcopy.h"
 
 #include <hip/hip_runtime.h>
 
@@ -25,6 +26,7 @@ struct lbm_cg_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void* P[2] = {nullptr, nullptr};
     int cur = 0;
+    int dev = 0;                 // device current at creation
     int64_t steps = -1;
     double* mac = nullptr;       // 6 N: rho_r, rho_b, rho, u, v, w
     double* rr0 = nullptr;       // 2 N initial densities
@@ -104,6 +106,8 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return LBM_EDEVICE;
     lbm_cg_ctx* c = new lbm_cg_ctx();
+    lbm::host_staging_retain();
+    (void)hipGetDevice(&c->dev);
     c->p = *p;
     c->n = n;
     c->q = q;
@@ -168,6 +172,7 @@ void lbm_cg_destroy(lbm_cg_ctx* c) {
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
     if (c->stream) hipStreamDestroy(c->stream);
+    lbm::host_staging_release();
     delete c;
 }
 
@@ -259,9 +264,11 @@ lbm_status lbm_cg_get_macros3d(lbm_cg_ctx* c, double* rr, double* rb, double* rh
     if (!c) return LBM_EINVAL;
     if (c->steps < 0) return cfail(c, LBM_EINVAL, "state not initialised");
     double* d[6] = {rr, rb, rho, u, v, w};
+    lbm::OutCopy out[6];
+    int n = 0;
     for (int a = 0; a < 6; ++a)
-        if (d[a]) CGCHK(c, hipMemcpyAsync(d[a], c->mac + a * c->n, 8 * c->n, hipMemcpyDeviceToHost, c->stream));
-    CGCHK(c, hipStreamSynchronize(c->stream));
+        if (d[a]) out[n++] = {d[a], c->mac + a * c->n, 8 * c->n};
+    CGCHK(c, lbm::copy_to_host(out, n, c->dev, c->stream));
     return LBM_OK;
 }
 
@@ -276,9 +283,8 @@ lbm_status lbm_cg_get_f(lbm_cg_ctx* c, double* rf, double* bf) {
         CGCHK(c, lbm::cg3_launch_recon(c->p.storage, c->P[c->cur ^ 1], c->cp, c->fout, c->fout + qn, c->stream));
     else
         CGCHK(c, lbm::cg_launch_recon(c->p.storage, c->P[c->cur ^ 1], c->cp, c->fout, c->fout + qn, c->stream));
-    CGCHK(c, hipMemcpyAsync(rf, c->fout, 8 * qn, hipMemcpyDeviceToHost, c->stream));
-    CGCHK(c, hipMemcpyAsync(bf, c->fout + qn, 8 * qn, hipMemcpyDeviceToHost, c->stream));
-    CGCHK(c, hipStreamSynchronize(c->stream));
+    const lbm::OutCopy out[2] = {{rf, c->fout, 8 * qn}, {bf, c->fout + qn, 8 * qn}};
+    CGCHK(c, lbm::copy_to_host(out, 2, c->dev, c->stream));
     return LBM_OK;
 }
 
