@@ -106,6 +106,10 @@ hipError_t cg_launch_reduce(const double* mac, size_t n, bool three_d, double ka
 // Pc after collision
 hipError_t cgw_launch_step(int storage, const void* P, void* Pc, double* mac, const cg::WallParams& wp,
                            hipStream_t st);
+// the D2Q9 step with FP64 storage: populations and macros after the wall
+// condition from P, mac to Pn, macn
+hipError_t cgw_launch_step64(const double* P, double* Pn, const double* mac, double* macn, const cg::WallParams& wp,
+                             hipStream_t st);
 hipError_t cgw_launch_init(int storage, void* P, double* mac, const double* rr, const double* rb, const double* rf,
                            const double* bf, const cg::WallParams& wp, hipStream_t st);
 hipError_t cgw_launch_out(int storage, int q, const void* P, size_t n, double* rf, double* bf, hipStream_t st);

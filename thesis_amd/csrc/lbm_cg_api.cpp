@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -29,11 +30,13 @@ struct lbm_cg_ctx {
     int dev = 0;                 // device current at creation
     int64_t steps = -1;
     double* mac = nullptr;       // 6 N: rho_r, rho_b, rho, u, v, w
+    double* mac2 = nullptr;      // the macros of the step before (fused_walls)
     double* rr0 = nullptr;       // 2 N initial densities
     void* psi = nullptr;         // 3 N phase field, density, red density (D3Q19)
     double* fout = nullptr;      // 2 q N: populations in and out
     double* partials = nullptr;
     bool walls = false;          // walls or body force: the reference-order path (lbm_cgw.hip)
+    bool fused_walls = false;    // of these D2Q9 FP64: one launch a step, from P[cur] and mac to P[cur ^ 1] and mac2
     lbm::cg::WallParams wp{};
     std::string err;
 };
@@ -141,6 +144,7 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
         }
     }
     c->walls = walls;
+    c->fused_walls = walls && !three_d && p->storage == LBM_STORE_F64;
     c->wp.cp = k;
     c->wp.walls = p->walls;
     c->wp.ho = p->high_order;
@@ -154,7 +158,9 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
          hipMalloc((void**)&c->mac, 6 * n * 8) == hipSuccess && hipMalloc((void**)&c->rr0, 2 * n * 8) == hipSuccess &&
          hipMalloc((void**)&c->partials, (size_t)kRedBlocks * lbm::cg::NRED * 8) == hipSuccess &&
          (!three_d || hipMalloc(&c->psi, 3 * n * 8) == hipSuccess) &&
-         hipMemset(c->mac + 5 * n, 0, n * 8) == hipSuccess;
+         hipMemset(c->mac + 5 * n, 0, n * 8) == hipSuccess &&
+         (!c->fused_walls || (hipMalloc((void**)&c->mac2, 6 * n * 8) == hipSuccess &&
+                              hipMemset(c->mac2 + 5 * n, 0, n * 8) == hipSuccess));
     if (!ok) {
         lbm_cg_destroy(c);
         return LBM_ENOMEM;
@@ -166,7 +172,7 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
 void lbm_cg_destroy(lbm_cg_ctx* c) {
     if (!c) return;
     if (c->stream) hipStreamSynchronize(c->stream);
-    void* b[] = {c->P[0], c->P[1], c->mac, c->rr0, c->psi, c->fout, c->partials};
+    void* b[] = {c->P[0], c->P[1], c->mac, c->mac2, c->rr0, c->psi, c->fout, c->partials};
     for (void* x : b)
         if (x) hipFree(x);
     if (c->ev0) hipEventDestroy(c->ev0);
@@ -230,6 +236,13 @@ lbm_status lbm_cg_init_f(lbm_cg_ctx* c, const double* r_f, const double* b_f) {
 static lbm_status cg_run(lbm_cg_ctx* c, int64_t nsteps) {
     for (int64_t k = 0; k < nsteps; ++k) {
         const bool wm = k == nsteps - 1;
+        if (c->fused_walls) {
+            CGCHK(c, lbm::cgw_launch_step64((const double*)c->P[c->cur], (double*)c->P[c->cur ^ 1], c->mac, c->mac2,
+                                            c->wp, c->stream));
+            std::swap(c->mac, c->mac2);
+            c->cur ^= 1;
+            continue;
+        }
         if (c->walls) {
             // P[0]: populations after the wall condition, P[1]: after collision
             CGCHK(c, lbm::cgw_launch_step(c->p.storage, c->P[0], c->P[1], c->mac, c->wp, c->stream));
@@ -278,7 +291,7 @@ lbm_status lbm_cg_get_f(lbm_cg_ctx* c, double* rf, double* bf) {
     const size_t qn = (size_t)c->q * c->n;
     if (!c->fout && hipMalloc((void**)&c->fout, 2 * qn * 8) != hipSuccess) return LBM_ENOMEM;
     if (c->walls)
-        CGCHK(c, lbm::cgw_launch_out(c->p.storage, c->q, c->P[0], c->n, c->fout, c->fout + qn, c->stream));
+        CGCHK(c, lbm::cgw_launch_out(c->p.storage, c->q, c->P[c->cur], c->n, c->fout, c->fout + qn, c->stream));
     else if (c->three_d)
         CGCHK(c, lbm::cg3_launch_recon(c->p.storage, c->P[c->cur ^ 1], c->cp, c->fout, c->fout + qn, c->stream));
     else

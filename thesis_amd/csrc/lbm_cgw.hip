@@ -29,6 +29,7 @@
 // (S/GpuUpdateMacro.cu:215-345).
 // Each thread reads its neighbours only from arrays the launch does not
 // write, and writes only its own node.
+// D2Q9 with FP64 storage does both halves in one launch (k_cgw_step64).
 #include "lbm_cg.h"
 #include "lbm_device.h"
 
@@ -227,6 +228,204 @@ __global__ __launch_bounds__(256) void k_cgw_stream(const T* __restrict__ Pc, T*
     mac[2 * n + ind] = (double)r;
     mac[3 * n + ind] = (double)(jx / r + (wp.external_force ? g / (r * om) : (T)0));
     mac[4 * n + ind] = (double)(jy / r + (wp.external_force ? (T)0 : g / om));
+}
+
+// The condition of a wall row on one colour, Zou-He velocity (walls 1, the two
+// functions above in one) or bounce-back; links chosen by value, so that the
+// array stays in registers.  Returns the colour's density of the first.
+__device__ inline double wall_row64(double (&f)[9], int walls, double u, double v, bool north) {
+    const double a = north ? f[2] : f[4], b = north ? f[5] : f[7], c = north ? f[6] : f[8];
+    double r = 0, da = 0, db = 0, dc = 0;
+    if (walls == 1) {
+        const double s = north ? 1.0 : -1.0, t = 0.5 * (f[1] - f[3]);
+        r = (f[0] + f[1] + f[3] + 2.0 * (a + b + c)) / (1.0 + s * v);
+        da = s * (-(2.0 / 3.0) * r * v);
+        db = s * (t - (1.0 / 6.0) * (r * v) - 0.5 * (r * u));
+        dc = s * (-t - (1.0 / 6.0) * (r * v) + 0.5 * (r * u));
+    }
+    f[4] = north ? a + da : f[4];
+    f[7] = north ? b + db : f[7];
+    f[8] = north ? c + dc : f[8];
+    f[2] = north ? f[2] : a + da;
+    f[5] = north ? f[5] : b + db;
+    f[6] = north ? f[6] : c + dc;
+    return r;
+}
+
+// One FP64 step in a single launch, populations and macros from one pair of
+// buffers to the other.
+//
+// A workgroup holds BX x BY nodes, one a thread, of which the (BX-2) x (BY-2)
+// inside the frame are its own: every thread reads its node's populations and
+// macros and collides, the moving links change hands through LDS, and the
+// inner threads pull them, apply the wall condition and store.  The weighted
+// phase field (and with E the density) of the nodes and of H more rings goes to
+// LDS, so that a node divides once for each weight instead of once for each
+// neighbour: one division with the 8-point stencil (4/12 is exactly four times
+// 1/12), five more with the 24-point one.  The sums keep gradient()'s terms and
+// order to the bit: with no g_limit, where the field is flat the direction of
+// what rounding leaves is what recolours the traces of the other fluid.  The
+// wall condition and the force shift take the stored macros and links from
+// registers.
+//
+// What bounds a box that fits the caches is one wavefront's chain of FP64
+// instructions (250 x 187: 47 k nodes, a wavefront a SIMD): the two launches
+// took 15.7 us a step there, this one 7.9 us.  Larger ones move 48 instead of 92
+// values a node: 1024 x 700 91 to 56 us.
+template <int BX, int BY, int H, bool E>
+__global__ __launch_bounds__(BX * BY) void k_cgw_step64(const double* __restrict__ P, double* __restrict__ Pn,
+                                                        const double* __restrict__ mac, double* __restrict__ macn,
+                                                        WallParams wp) {
+    constexpr int NT = BX * BY, RW = BX + 2 * H, RH = BY + 2 * H;
+    constexpr int C2[6] = {0, 1, 2, 4, 5, 8};   // |c|^2 of the 24-point stencil's weights
+    __shared__ double psi[H == 1 ? 1 : 6][RW * RH];
+    __shared__ double rt[E ? RW * RH : 1];
+    __shared__ double ex[16][NT];   // moving links after collision, red then blue
+    const CgParams& cp = wp.cp;
+    const int nx = cp.nx, ny = cp.ny;
+    const uint32_t n = (uint32_t)nx * (uint32_t)ny;
+    const int tid = threadIdx.x, tx = tid % BX, ty = tid / BX;
+    const uint32_t b = xcd_block(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y, cp.xcd_shift,
+                                 cp.xchunk_shift);
+    const uint32_t by = b / gridDim.x;
+    // node of thread (0, 0)
+    const int x0 = (int)(b - by * gridDim.x) * (BX - 2) - 1, y0 = (int)by * (BY - 2) - 1;
+    // rows beyond a wall read the wall row: nothing made from them is kept
+    auto pwrap = [](int a, int m) { return a >= 0 && a < m ? a : ((a % m) + m) % m; };
+    auto row = [&](int a) { return wp.walls ? (a < 0 ? 0 : (a >= ny ? ny - 1 : a)) : pwrap(a, ny); };
+    const int x = pwrap(x0 + tx, nx), y = row(y0 + ty);
+    const bool beyond = wp.walls && y != y0 + ty;
+    auto field = [&](int j, double d, double rho) {
+        psi[0][j] = (1.0 / 12.0) * d / rho;
+        if (H == 2) {
+#pragma unroll
+            for (int c = 1; c < 6; ++c) psi[H == 1 ? 0 : c][j] = HOW(C2[c]) * d / rho;
+        }
+        if (E) rt[j] = rho;
+    };
+    const uint32_t ind = (uint32_t)y * (uint32_t)nx + (uint32_t)x;
+    const double rr = mac[ind], br = mac[n + ind], r = mac[2 * n + ind];
+    const double u = mac[3 * n + ind], v = mac[4 * n + ind];
+    double fr[9], fb[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        fr[k] = P[(size_t)k * n + ind];
+        fb[k] = P[(size_t)(9 + k) * n + ind];
+    }
+    for (int e = tid; e < RW * RH - NT; e += NT) {
+        int px, py;   // top H rows, bottom H rows, then the H columns left and right
+        if (e < H * RW) { py = e / RW; px = e % RW; }
+        else if (e < 2 * H * RW) { const int q = e - H * RW; py = BY + H + q / RW; px = q % RW; }
+        else { const int q = e - 2 * H * RW, c = q % (2 * H); py = H + q / (2 * H); px = c < H ? c : BX + c; }
+        const uint32_t j = (uint32_t)row(y0 + py - H) * (uint32_t)nx + (uint32_t)pwrap(x0 + px - H, nx);
+        field(py * RW + px, mac[j] - mac[n + j], mac[2 * n + j]);
+    }
+    const double ir = 1.0 / r;
+    const int at = (ty + H) * RW + tx + H;
+    field(at, rr - br, r);
+    __syncthreads();
+
+    const bool wall_row = wp.walls && (y == 0 || y == ny - 1);
+    const bool north = y == ny - 1;
+    double gx = 0, gy = 0, dx = 0, dy = 0;
+    if (!beyond) {
+        auto take = [&](int j, double p, double w, int kx, int ky) {
+            if (kx) gx += kx * p;
+            if (ky) gy += ky * p;
+            if (E) {
+                const double q = w * rt[j];
+                if (kx) dx += kx * q;
+                if (ky) dy += ky * q;
+            }
+        };
+        if (H == 1 || wall_row || (wp.walls && (y == 1 || y == ny - 2))) {
+            // on a wall row the rows beyond the wall are mirrored onto the row
+            // inside and only the x components are taken
+            const int up = wall_row && north ? -RW : RW, down = wall_row && !north ? RW : -RW;
+#pragma unroll
+            for (int k = 1; k < 9; ++k) {
+                const int j = at + CX[k] + (CY[k] > 0 ? up : CY[k] < 0 ? down : 0);
+                take(j, k < 5 ? 4.0 * psi[0][j] : psi[0][j], k < 5 ? 4.0 / 12.0 : 1.0 / 12.0, CX[k], CY[k]);
+            }
+            if (wall_row) gy = dy = 0;
+        } else {
+#pragma unroll
+            for (int ddy = -H; ddy <= H; ++ddy)
+#pragma unroll
+                for (int ddx = -H; ddx <= H; ++ddx) {
+                    const int c2 = ddx * ddx + ddy * ddy, j = at + ddy * RW + ddx;
+                    const int c = c2 == 8 ? 5 : c2 == 5 ? 4 : c2 == 4 ? 3 : c2;
+                    if (c2) take(j, psi[H == 1 ? 0 : c][j], HOW(c2), ddx, ddy);
+                }
+        }
+    }
+    const double kr = rr * ir, kb = br * ir, kk = cp.beta * rr * kb;
+    const double mean_nu = (cp.r_nu * cp.b_nu) / (kr * cp.b_nu + kb * cp.r_nu);
+    double iom = 3.0 * mean_nu + 0.5;
+    const double om = 1.0 / iom, alpha = cp.r_alpha * kr + cp.b_alpha * kb;
+    const double gn = sqrt(gx * gx + gy * gy);
+    const bool on = gn > cp.g_limit;
+    const double ign = on ? 1.0 / gn : 0.0;
+    const double ag = on ? cp.A * gn : 0.0, nxg = gx * ign, nyg = gy * ign;
+    const double uu = u * u + v * v, ugr = u * dx + v * dy;
+    double f0r = 0, f0b = 0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        // c_k . grad / |grad|; its square is the perturbation's, over |c_k| the recolouring's
+        const double cn = cg::cdot<double>(CX[k], CY[k], 0, nxg, nyg, 0.0);
+        const double cs = k ? cn * (1.0 / CNORM(k)) : 0.0;
+        const double pert = ag * (W9(k) * cn * cn - BPERT(k));
+        const double cu = cg::cdot<double>(CX[k], CY[k], 0, u, v, 0.0);
+        const double rest = PHI(k) + TETA(k) * alpha;
+        double feq = r * (rest + W9(k) * (3.0 * cu + 4.5 * cu * cu - 1.5 * uu));
+        if (E) {
+            const double cgr = cg::cdot<double>(CX[k], CY[k], 0, dx, dy, 0.0);
+            feq += mean_nu * (CHI(k) * ugr + PSI(k) * 2.0 * cu * cgr);
+        }
+        const double fs = om * feq + (1.0 - om) * (fr[k] + fb[k]) + pert;
+        const double cr = kr * fs + kk * cs * rest, cb = kb * fs - kk * cs * rest;
+        if (k) { ex[k - 1][tid] = cr; ex[7 + k][tid] = cb; }
+        else { f0r = cr; f0b = cb; }
+    }
+    __syncthreads();
+
+    if (tx < 1 || tx >= BX - 1 || ty < 1 || ty >= BY - 1 || x0 + tx >= nx || y0 + ty >= ny) return;
+    fr[0] = f0r;
+    fb[0] = f0b;
+#pragma unroll
+    for (int k = 1; k < 9; ++k) {
+        // a wall row keeps its links from beyond the wall; the condition sets them
+        const bool keep = wall_row && (CY[k] > 0 ? !north : CY[k] < 0 && north);
+        const int j = tid - CX[k] - BX * CY[k];
+        const double cr = ex[k - 1][j], cb = ex[7 + k][j];
+        fr[k] = keep ? fr[k] : cr;
+        fb[k] = keep ? fb[k] : cb;
+    }
+    if (wall_row) {
+        const double rr0 = wall_row64(fr, wp.walls, u, v, north), br0 = wall_row64(fb, wp.walls, u, v, north);
+        if (wp.walls == 1) {
+            const double r0 = rr0 + br0;
+            iom = 3.0 / (rr0 / (r0 * cp.r_nu) + br0 / (r0 * cp.b_nu)) + 0.5;
+        }
+    }
+    double R = 0, B = 0, jx = 0, jy = 0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        Pn[(size_t)k * n + ind] = fr[k];
+        Pn[(size_t)(9 + k) * n + ind] = fb[k];
+        R += fr[k];
+        B += fb[k];
+        const double f = fr[k] + fb[k];
+        if (CX[k]) jx += CX[k] > 0 ? f : -f;
+        if (CY[k]) jy += CY[k] > 0 ? f : -f;
+    }
+    // 1 / omega_eff from the densities stored before this update (S/GpuUpdateMacro.cu:62-64)
+    const double rn = R + B, irn = 1.0 / rn, gs = wp.g * iom;
+    macn[ind] = R;
+    macn[n + ind] = B;
+    macn[2 * n + ind] = rn;
+    macn[3 * n + ind] = jx * irn + (wp.external_force ? gs * irn : 0.0);
+    macn[4 * n + ind] = jy * irn + (wp.external_force ? 0.0 : gs);
 }
 
 // Rest-state colours from colour densities (S/GpuInit.cu:323-352), or given
@@ -497,25 +696,35 @@ hipError_t cgw_launch_step(int storage, const void* P, void* Pc, double* mac, co
 #undef CGW3_
         return hipGetLastError();
     }
-    if (storage == 0) {
-        if (wp.cp.enhanced)
-            hipLaunchKernelGGL((cgw::k_cgw_collide<double, true>), dim3(blocks), dim3(256), 0, st, (const double*)P,
-                               (double*)Pc, mac, wp);
-        else
-            hipLaunchKernelGGL((cgw::k_cgw_collide<double, false>), dim3(blocks), dim3(256), 0, st, (const double*)P,
-                               (double*)Pc, mac, wp);
-        hipLaunchKernelGGL(cgw::k_cgw_stream<double>, dim3(blocks), dim3(256), 0, st, (const double*)Pc, (double*)P,
-                           mac, wp);
-    } else {
-        if (wp.cp.enhanced)
-            hipLaunchKernelGGL((cgw::k_cgw_collide<float, true>), dim3(blocks), dim3(256), 0, st, (const float*)P,
-                               (float*)Pc, mac, wp);
-        else
-            hipLaunchKernelGGL((cgw::k_cgw_collide<float, false>), dim3(blocks), dim3(256), 0, st, (const float*)P,
-                               (float*)Pc, mac, wp);
-        hipLaunchKernelGGL(cgw::k_cgw_stream<float>, dim3(blocks), dim3(256), 0, st, (const float*)Pc, (float*)P, mac,
-                           wp);
-    }
+    // D2Q9 here: FP32 (FP64 goes by cgw_launch_step64)
+    if (wp.cp.enhanced)
+        hipLaunchKernelGGL((cgw::k_cgw_collide<float, true>), dim3(blocks), dim3(256), 0, st, (const float*)P,
+                           (float*)Pc, mac, wp);
+    else
+        hipLaunchKernelGGL((cgw::k_cgw_collide<float, false>), dim3(blocks), dim3(256), 0, st, (const float*)P,
+                           (float*)Pc, mac, wp);
+    hipLaunchKernelGGL(cgw::k_cgw_stream<float>, dim3(blocks), dim3(256), 0, st, (const float*)Pc, (float*)P, mac, wp);
+    return hipGetLastError();
+}
+
+hipError_t cgw_launch_step64(const double* P, double* Pn, const double* mac, double* macn, const cg::WallParams& wp,
+                             hipStream_t st) {
+#define CGW64(BX_, BY_, H_, E_)                                                                                  \
+    hipLaunchKernelGGL((cgw::k_cgw_step64<BX_, BY_, H_, E_>),                                                    \
+                       dim3((wp.cp.nx + BX_ - 3) / (BX_ - 2), (wp.cp.ny + BY_ - 3) / (BY_ - 2)), dim3(BX_ * BY_), 0, \
+                       st, P, Pn, mac, macn, wp)
+#define CGW64_E(BX_, BY_, H_) \
+    do { if (wp.cp.enhanced) CGW64(BX_, BY_, H_, true); else CGW64(BX_, BY_, H_, false); } while (0)
+    // Small workgroups fill the chip on small boxes (250 x 187: 7.9 us with
+    // 16 x 16, 8.5 us with 32 x 16) and leave room for the 24-point stencil's
+    // fields in LDS (512 x 512: 24.3 against 27.2 us); from 2^18 nodes the
+    // 8-point step is bound by its traffic and the larger one reads a smaller
+    // frame (512 x 512: 20.1 against 21.1 us, 1024 x 700: 56 against 65 us).
+    if (wp.ho) CGW64_E(16, 16, 2);
+    else if ((size_t)wp.cp.nx * wp.cp.ny < (size_t)1 << 18) CGW64_E(16, 16, 1);
+    else CGW64_E(32, 16, 1);
+#undef CGW64_E
+#undef CGW64
     return hipGetLastError();
 }
 
