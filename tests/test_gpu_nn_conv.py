@@ -107,6 +107,22 @@ def test_grad_sum(N, M):
         assert torch.equal(got, want) and torch.equal(gb, wb)
 
 
+def test_rounding_of_special_values():
+    """Ties, values next to them, the smallest, the largest and infinities round as
+    the integer rounding of grad_bf16 does; NaN stays NaN."""
+    hi = np.arange(0, 1 << 16, 7, dtype=np.uint32)
+    words = (hi[:, None] << 16 | np.array([0, 1, 0x7FFF, 0x8000, 0x8001, 0x8003, 0xFFFF], np.uint32)).ravel()
+    words = np.concatenate([words, np.array([0x7F800000, 0xFF800000, 0x7F7FFFFF, 1, 0x7F800001, 0x7FFFFFFF], np.uint32)])
+    words = np.resize(words, (words.size + 31) // 32 * 32)
+    dy, n = dev(words.view(np.float32)), words.size
+    want, got, db = i16(n), i16(n), torch.zeros(32, device=DEV)
+    nn.grad_bf16(dy, dy, 0, want)
+    nn.grad_sum(dy, dy, 0, 32, got, db)
+    nan = np.isnan(words.view(np.float32))
+    w, g = want.cpu().numpy(), got.cpu().numpy()
+    assert np.array_equal(w[~nan], g[~nan]) and ((g[nan] & 0x7FFF) > 0x7F80).all()
+
+
 def test_refused_shapes():
     z, w = f32(64), i16(64)
     for cin, cout, k, mode in ((5, 32, 3, 0), (32, 48, 3, 0), (32, 33, 1, 0), (32, 32, 3, 1), (32, 32, 3, 2)):

@@ -8,10 +8,13 @@
 // read from L2 (each wave's own columns; 18-295 KB a layer).  One LDS read of
 // a pixel serves nine taps, where im2col wrote and read it nine times.
 //
-// Prediction of 8 channels of 512 x 128: 3.11 -> 0.69 ms against im2col (55 % of
+// Prediction of 8 channels of 512 x 128: 3.11 -> 0.63 ms against im2col (55 % of
 // the time) + GEMM + upsampling and skip-sum passes; a training step on 16:
-// 21.4 -> 4.5 ms.  What bounds it now: the FP32 activations' traffic at full
-// resolution (32 channels), the MFMA at the coarse levels.
+// 21.4 -> 3.9 ms.  What bounds it now: the FP32 activations' traffic at full
+// resolution (32 channels); at the coarse levels the latency of staging and
+// weights, one or two workgroups a CU (128 channels: 34 us of which 8 are MFMA).
+// Weights staged in LDS for the four waves cost more in barriers and in
+// workgroups a CU than they saved (43 us), loads six steps ahead gave nothing.
 //
 // The sums run in the order of the im2col GEMM (tap, then channel, 16 at a time
 // in v_mfma_f32_32x32x16_bf16), so outputs are the same bits.
@@ -31,13 +34,12 @@ typedef uint16_t u16;
 
 constexpr int TX = 32;   // pixels of a tile row: the 32 rows of an MFMA operand
 
-__device__ inline u16 f2bf(float f) {   // round to nearest even
-    const uint32_t u = __float_as_uint(f);
-    if ((u & 0x7F800000u) == 0x7F800000u) return (u16)((u >> 16) | ((u & 0xFFFFu) ? 0x40u : 0u));
-    return (u16)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
+// Rounded to nearest even by v_cvt_pk_bf16_f32: half an instruction a value, where
+// the same rounding in integer arithmetic took about eight and the staging of a
+// tile as long as its MFMA.
 __device__ inline uint2 f2bf4(f32x4 v) {
-    return make_uint2(f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16, f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16);
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(uint2, bf16x4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]});
 }
 
 // Input of a convolution: x itself, x at half the resolution (each pixel read by
@@ -61,45 +63,80 @@ __device__ inline f32x4 fetch(const Img& s, int b, int y, int x, int c) {
     return v;
 }
 
+// The staging loops below load from the nearest pixel inside the image and zero
+// what lies outside after the load, U loads of a thread at a time: a load under a
+// branch would be waited for before the next is issued (weight gradients of a
+// training step 1.55 -> 0.99 ms, forward convolutions of a prediction 0.64 -> 0.57).
+__device__ inline int clampi(int a, int n) { return a < 0 ? 0 : (a >= n ? n - 1 : a); }
+
 // Channels c0 .. c0+KC-1 of the ROWS x COLS pixels at (y0, x0) as bf16 in LDS,
 // zero outside the image; pitch P.
-template <int KC, int P, int ROWS, int COLS, int MODE>
+template <int KC, int P, int ROWS, int COLS, int MODE, int U>
 __device__ inline void stage(const Img& s, int b, int y0, int x0, int c0, u16* t) {
-    constexpr int V = KC / 4, N = ROWS * COLS * V;
-#pragma unroll 4
-    for (int v = threadIdx.x; v < N; v += 256) {
-        const int px = v / V, c = (v - px * V) * 4, r = px / COLS;
-        const int y = y0 + r, x = x0 + px - r * COLS;
-        uint2 e = make_uint2(0u, 0u);
-        if (y >= 0 && y < s.H && x >= 0 && x < s.W) e = f2bf4(fetch<MODE>(s, b, y, x, c0 + c));
-        *(uint2*)(t + px * P + c) = e;
+    constexpr int V = KC / 4, N = ROWS * COLS * V, NV = (N + 255) / 256;
+    for (int i0 = 0; i0 < NV; i0 += U) {
+        f32x4 e[U];
+        bool in[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v0 = threadIdx.x + 256 * (i0 + i), v = v0 < N ? v0 : N - 1;
+            const int px = v / V, c = (v - px * V) * 4, r = px / COLS;
+            const int y = y0 + r, x = x0 + px - r * COLS;
+            in[i] = y >= 0 && y < s.H && x >= 0 && x < s.W;
+            e[i] = fetch<MODE>(s, b, clampi(y, s.H), clampi(x, s.W), c0 + c);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v = threadIdx.x + 256 * (i0 + i), px = v / V, c = (v - px * V) * 4;
+            const uint2 q = f2bf4(e[i]);
+            if (v < N) *(uint2*)(t + px * P + c) = in[i] ? q : make_uint2(0u, 0u);
+        }
     }
 }
 // The same of a bf16 image (8 channels a load).
-template <int KC, int P, int ROWS, int COLS>
+template <int KC, int P, int ROWS, int COLS, int U>
 __device__ inline void stage_bf(const u16* __restrict__ z, int H, int W, int C, int b, int y0, int x0, int c0, u16* t) {
-    constexpr int V = KC / 8, N = ROWS * COLS * V;
-#pragma unroll 4
-    for (int v = threadIdx.x; v < N; v += 256) {
-        const int px = v / V, c = (v - px * V) * 8, r = px / COLS;
-        const int y = y0 + r, x = x0 + px - r * COLS;
-        uint4 e = make_uint4(0u, 0u, 0u, 0u);
-        if (y >= 0 && y < H && x >= 0 && x < W) e = *(const uint4*)(z + (((size_t)b * H + y) * W + x) * C + c0 + c);
-        *(uint4*)(t + px * P + c) = e;
+    constexpr int V = KC / 8, N = ROWS * COLS * V, NV = (N + 255) / 256;
+    for (int i0 = 0; i0 < NV; i0 += U) {
+        uint4 e[U];
+        bool in[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v0 = threadIdx.x + 256 * (i0 + i), v = v0 < N ? v0 : N - 1;
+            const int px = v / V, c = (v - px * V) * 8, r = px / COLS;
+            const int y = y0 + r, x = x0 + px - r * COLS;
+            in[i] = y >= 0 && y < H && x >= 0 && x < W;
+            e[i] = *(const uint4*)(z + (((size_t)b * H + clampi(y, H)) * W + clampi(x, W)) * C + c0 + c);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v = threadIdx.x + 256 * (i0 + i), px = v / V, c = (v - px * V) * 8;
+            if (v < N) *(uint4*)(t + px * P + c) = in[i] ? e[i] : make_uint4(0u, 0u, 0u, 0u);
+        }
     }
 }
 // Four input channels: the nine taps of a pixel side by side (36 of KC columns,
 // the rest zero), so that the patch is a matrix row per pixel.
-template <int KC, int P, int ROWS>
+template <int KC, int P, int ROWS, int U>
 __device__ inline void stage_taps(const Img& s, int b, int y0, int x0, u16* t) {
-    constexpr int V = KC / 4, N = ROWS * TX * V;
-#pragma unroll 4
-    for (int v = threadIdx.x; v < N; v += 256) {
-        const int px = v / V, tap = v - px * V, r = px / TX, ky = tap / 3;
-        const int y = y0 + r + ky - 1, x = x0 + px - r * TX + (tap - 3 * ky) - 1;
-        uint2 e = make_uint2(0u, 0u);
-        if (tap < 9 && y >= 0 && y < s.H && x >= 0 && x < s.W) e = f2bf4(fetch<IN_X>(s, b, y, x, 0));
-        *(uint2*)(t + px * P + tap * 4) = e;
+    constexpr int V = KC / 4, N = ROWS * TX * V, NV = (N + 255) / 256;
+    for (int i0 = 0; i0 < NV; i0 += U) {
+        f32x4 e[U];
+        bool in[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v0 = threadIdx.x + 256 * (i0 + i), v = v0 < N ? v0 : N - 1;
+            const int px = v / V, tap = v - px * V, r = px / TX, ky = tap / 3;
+            const int y = y0 + r + ky - 1, x = x0 + px - r * TX + (tap - 3 * ky) - 1;
+            in[i] = tap < 9 && y >= 0 && y < s.H && x >= 0 && x < s.W;
+            e[i] = fetch<IN_X>(s, b, clampi(y, s.H), clampi(x, s.W), 0);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v = threadIdx.x + 256 * (i0 + i), px = v / V, tap = v - px * V;
+            const uint2 q = f2bf4(e[i]);
+            if (v < N) *(uint2*)(t + px * P + tap * 4) = in[i] ? q : make_uint2(0u, 0u);
+        }
     }
 }
 
@@ -124,8 +161,8 @@ __global__ __launch_bounds__(256) void k_conv(Img s, const u16* __restrict__ w, 
     __shared__ __align__(16) u16 t[ROWS * COLS * P];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / WN, wn = wave % WN;
     const Tile tl = tile_of(blockIdx.x, tx, ty, TY);
-    if (KIND == 1) stage_taps<KC, P, ROWS>(s, tl.b, tl.y0, tl.x0, t);
-    else stage<KC, P, ROWS, COLS, MODE>(s, tl.b, tl.y0 - HALO, tl.x0 - HALO, 0, t);
+    if (KIND == 1) stage_taps<KC, P, ROWS, 6>(s, tl.b, tl.y0, tl.x0, t);
+    else stage<KC, P, ROWS, COLS, MODE, MODE == IN_ADD ? 4 : 8>(s, tl.b, tl.y0 - HALO, tl.x0 - HALO, 0, t);
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -200,7 +237,7 @@ __global__ __launch_bounds__(256) void k_conv_dx(const u16* __restrict__ dz, int
     __shared__ __align__(16) u16 t[ROWS * COLS * P];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / WN, wn = wave % WN;
     const Tile tl = tile_of(blockIdx.x, tx, ty, TY);
-    stage_bf<KC, P, ROWS, COLS>(dz, H, W, KC, tl.b, tl.y0 - 1, tl.x0 - 1, 0, t);
+    stage_bf<KC, P, ROWS, COLS, 6>(dz, H, W, KC, tl.b, tl.y0 - 1, tl.x0 - 1, 0, t);
     f32x16 tot[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -284,7 +321,7 @@ __device__ inline bf16x8 read_tr(const u16* t, int lane) {
 // with one atomic per weight.  KIND as in k_conv (1: the 64 columns of nine taps
 // of four channels in two blocks of 32).
 template <int KIND, int MODE>
-__global__ __launch_bounds__(256) void k_conv_dw(Img s, const u16* __restrict__ dz, int N, int kp, uint32_t tx,
+__global__ __launch_bounds__(256, 2) void k_conv_dw(Img s, const u16* __restrict__ dz, int N, int kp, uint32_t tx,
                                                  uint32_t ty, uint32_t ntiles, int ncb, float* __restrict__ dw) {
     constexpr int TY = 8, HALO = KIND == 0 ? 1 : 0, COLS = TX + 2 * HALO, ROWS = TY + 2 * HALO;
     constexpr int TAPS = KIND == 0 ? 9 : 1, KC = KIND == 1 ? 64 : 32;
@@ -302,15 +339,17 @@ __global__ __launch_bounds__(256) void k_conv_dw(Img s, const u16* __restrict__ 
     for (uint32_t it = blockIdx.x; it < ntiles; it += gridDim.x) {
         const Tile tl = tile_of(it, tx, ty, TY);
         __syncthreads();   // the last tile's reads
-        if (KIND == 1) stage_taps<KC, KC, ROWS>(s, tl.b, tl.y0, tl.x0, t);
-        else stage<KC, KC, ROWS, COLS, MODE>(s, tl.b, tl.y0 - HALO, tl.x0 - HALO, c0, t);
+        if (KIND == 1) stage_taps<KC, KC, ROWS, 8>(s, tl.b, tl.y0, tl.x0, t);
+        else stage<KC, KC, ROWS, COLS, MODE, MODE == IN_ADD ? 4 : 6>(s, tl.b, tl.y0 - HALO, tl.x0 - HALO, c0, t);
         if (KIND == 2) {   // N < 32 columns, the rest zero
+#pragma unroll 8
             for (int v = threadIdx.x; v < ZT; v += 256) {
                 const int px = v >> 5, n = v & 31, y = tl.y0 + px / TX, x = tl.x0 + px % TX;
-                z[v] = n < N && y < s.H && x < s.W ? dz[(((size_t)tl.b * s.H + y) * s.W + x) * N + n] : (u16)0;
+                const u16 q = dz[(((size_t)tl.b * s.H + clampi(y, s.H)) * s.W + clampi(x, s.W)) * N + (n < N ? n : 0)];
+                z[v] = n < N && y < s.H && x < s.W ? q : (u16)0;
             }
         } else {
-            stage_bf<32, 32, TY, TX>(dz, s.H, s.W, N, tl.b, tl.y0, tl.x0, n0, z);
+            stage_bf<32, 32, TY, TX, 4>(dz, s.H, s.W, N, tl.b, tl.y0, tl.x0, n0, z);
         }
         __syncthreads();
 #pragma unroll
@@ -486,8 +525,9 @@ int nn_conv_dw(const float* x, const float* skip, int mode, const void* dz, int 
     const Img s{x, skip, H, W, cin};
     const uint32_t tx = (uint32_t)(W + TX - 1) / TX, ty = (uint32_t)(H + 7) / 8, nt = tx * ty * (uint32_t)Bn;
     const int ncb = taps4 ? 2 : cin / 32, pairs = ncb * ((cout + 31) / 32);
-    // two workgroups a CU over all channel pairs
-    const uint32_t gx = std::max(1u, std::min(nt, 512u / (uint32_t)pairs));
+    // two workgroups a CU over all channel pairs (nine accumulators a wave), three
+    // where one accumulator leaves the room
+    const uint32_t gx = std::max(1u, std::min(nt, (taps4 || one ? 768u : 512u) / (uint32_t)pairs));
     hipStream_t st = (hipStream_t)stream;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(gx, pairs), dim3(256), 0, st, s, (const u16*)dz, cout, kp, tx, ty, nt, ncb, dw);
