@@ -56,8 +56,10 @@ int nn_conv_dw(const float* x, const float* skip, int mode, const void* dz, int 
 /* per layer i < nlayers (at most 16): wt[to[i] + (tap*cin + c)*cout + n] = w[from[i] + n*kp + tap*cin + c] */
 int nn_weight_t(const void* w, int nlayers, const int64_t* from, const int64_t* to, const int* cin, const int* cout,
                 const int* kp, void* wt, void* stream);
-/* nn_grad_bf16 and nn_colsum in one pass (N 32, 64 or 128) */
-int nn_grad_sum(const float* dy, const float* y, int64_t n, int relu, int N, void* dz, float* db, void* stream);
+/* nn_grad_bf16 and nn_colsum in one pass (N 32, 64 or 128) over the Bn x H x W x N gradient that is dy (mode 0), the
+ * adjoint of nn_up2 on dy at 2H x 2W (1), or the adjoint of nn_avgpool2 on dy at H/2 x W/2, plus skip (2) */
+int nn_grad_sum(const float* dy, const float* skip, int mode, int Bn, int H, int W, const float* y, int relu, int N,
+                void* dz, float* db, void* stream);
 /* 2x2 average pooling and nearest x2 upsampling with their adjoints */
 int nn_avgpool2(const float* x, int Bn, int H, int W, int C, float* y, void* stream);
 int nn_avgpool2_bwd(const float* dy, int Bn, int H, int W, int C, float* dx, void* stream);

@@ -107,6 +107,25 @@ def test_grad_sum(N, M):
         assert torch.equal(got, want) and torch.equal(gb, wb)
 
 
+@pytest.mark.parametrize("N", [32, 64, 128])
+@pytest.mark.parametrize("B,H,W", [(1, 2, 2), (3, 6, 10), (2, 64, 34)])
+def test_grad_sum_through_upsampling_and_pooling(N, B, H, W):
+    """The same bits as the adjoint's own pass, then the plain gradient."""
+    r, n = rng(N + H), B * H * W * N
+    y, skip = dev(r.standard_normal(n)), dev(exact(r, n))
+    for mode, m in ((nn.GRAD_UP, 4 * n), (nn.GRAD_POOL, n // 4)):
+        dy, g = dev(exact(r, m)), f32(n)
+        if mode == nn.GRAD_UP:
+            nn.up2_bwd(dy, B, H, W, N, g)
+        else:
+            nn.avgpool2_bwd(dy, B, H, W, N, g)
+            nn.axpy(1.0, skip, g)
+        want, got, wb, gb = i16(n), i16(n), torch.ones(N, device=DEV), torch.ones(N, device=DEV)
+        nn.grad_sum(g, y, 1, N, want, wb)
+        nn.grad_sum(dy, y, 1, N, got, gb, mode, skip, (B, H, W))
+        assert torch.equal(got, want) and torch.equal(gb, wb)
+
+
 def test_rounding_of_special_values():
     """Ties, values next to them, the smallest, the largest and infinities round as
     the integer rounding of grad_bf16 does; NaN stays NaN."""

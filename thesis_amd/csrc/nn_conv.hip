@@ -10,7 +10,7 @@
 //
 // Prediction of 8 channels of 512 x 128: 3.11 -> 0.63 ms against im2col (55 % of
 // the time) + GEMM + upsampling and skip-sum passes; a training step on 16:
-// 21.4 -> 3.9 ms.  What bounds it now: the FP32 activations' traffic at full
+// 21.4 -> 3.4 ms.  What bounds it now: the FP32 activations' traffic at full
 // resolution (32 channels); at the coarse levels the latency of staging and
 // weights, one or two workgroups a CU (128 channels: 34 us of which 8 are MFMA).
 // Weights staged in LDS for the four waves cost more in barriers and in
@@ -382,14 +382,44 @@ __global__ __launch_bounds__(256, 2) void k_conv_dw(Img s, const u16* __restrict
     }
 }
 
-// dz = dy (times y > 0 when relu) as bf16 and its column sums, added to db:
-// one pass over dy and y, four channels a thread.  N (32, 64 or 128) divides the
-// 1024 values a workgroup covers, so a thread keeps its four columns.
-__global__ __launch_bounds__(256) void k_grad_sum(const float* __restrict__ dy, const float* __restrict__ y, int relu,
-                                                  size_t n4, int N, u16* __restrict__ dz, float* __restrict__ db) {
+// dz = g (times y > 0 when relu) as bf16 and its column sums, added to db, four
+// channels a thread.  The gradient g of the H x W image is dy itself; or the 2 x 2
+// sums of dy at twice the resolution (the adjoint of the upsampling); or dy at half
+// the resolution spread over 2 x 2 / 4, plus skip (the adjoint of the pooling, and
+// the gradient that came by the skip connection).  Nothing but this pass reads
+// such a g, so it is not stored.  N (32, 64 or 128) divides the 1024 values a
+// workgroup covers, so a thread keeps its four columns.
+//
+// Bound by its traffic; with the adjoints in passes of their own the backward of
+// 16 images of 512 x 128 spent 1.03 ms on all of them, now 0.63 ms.
+enum { GRAD_X = 0, GRAD_UP = 1, GRAD_POOL = 2 };
+template <int MODE>
+__global__ __launch_bounds__(256) void k_grad_sum(const float* __restrict__ dy, const float* __restrict__ skip,
+                                                  const float* __restrict__ y, int relu, uint32_t W, size_t n4, int N,
+                                                  u16* __restrict__ dz, float* __restrict__ db) {
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    const uint32_t n1 = (uint32_t)N / 4;
+#pragma unroll 2
     for (size_t e = blockIdx.x * (size_t)256 + threadIdx.x; e < n4; e += (size_t)gridDim.x * 256) {
-        f32x4 g = *(const f32x4*)(dy + 4 * e);
+        f32x4 g;
+        if (MODE == GRAD_X) {
+            g = *(const f32x4*)(dy + 4 * e);
+        } else {   // n4 is below 2^31
+            const uint32_t p = (uint32_t)e / n1, c = 4 * ((uint32_t)e - p * n1), row = p / W, x = p - row * W;
+            if (MODE == GRAD_UP) {
+                const float* q = dy + ((size_t)(2 * row) * (2 * W) + 2 * x) * N + c;
+                const size_t down = (size_t)2 * W * N;
+                const f32x4 a = *(const f32x4*)q, b = *(const f32x4*)(q + N);
+                const f32x4 d = *(const f32x4*)(q + down), f = *(const f32x4*)(q + down + N);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) g[i] = a[i] + b[i] + d[i] + f[i];
+            } else {
+                const f32x4 a = *(const f32x4*)(dy + ((size_t)(row >> 1) * (W >> 1) + (x >> 1)) * N + c);
+                const f32x4 b = *(const f32x4*)(skip + 4 * e);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) g[i] = 0.25f * a[i] + b[i];
+            }
+        }
         if (relu) {
             const f32x4 v = *(const f32x4*)(y + 4 * e);
 #pragma unroll
@@ -540,12 +570,23 @@ int nn_conv_dw(const float* x, const float* skip, int mode, const void* dz, int 
     return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
-int nn_grad_sum(const float* dy, const float* y, int64_t n, int relu, int N, void* dz, float* db, void* stream) {
-    if (n < 0 || (N != 32 && N != 64 && N != 128) || n % N || !aligned16(dz)) return 3;
-    if (n == 0) return 0;
-    const size_t n4 = (size_t)n / 4, blocks = std::min<size_t>(1024, (n4 + 255) / 256);
-    hipLaunchKernelGGL(k_grad_sum, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, dy, y, relu, n4, N,
-                       (u16*)dz, db);
+int nn_grad_sum(const float* dy, const float* skip, int mode, int Bn, int H, int W, const float* y, int relu, int N,
+                void* dz, float* db, void* stream) {
+    if (Bn < 0 || H < 1 || W < 1 || (N != 32 && N != 64 && N != 128) || !aligned16(dz)) return 3;
+    if (mode < 0 || mode > 2 || (mode == GRAD_POOL && (!skip || ((H | W) & 1)))) return 3;
+    if (mode != GRAD_X && !fits(Bn, H, W, N)) return 3;
+    if (Bn == 0) return 0;
+    // 512 workgroups: the column sums' atomics meet on N addresses (the training
+    // step's passes over 16 images take 0.63 ms with 512, 0.66 with 1024, 0.84 with
+    // 2048 and 256)
+    const size_t n4 = (size_t)Bn * H * W * N / 4, blocks = std::min<size_t>(512, (n4 + 255) / 256);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, dy, skip, y, relu,
+                           (uint32_t)W, n4, N, (u16*)dz, db);
+    };
+    if (mode == GRAD_UP) go(k_grad_sum<GRAD_UP>);
+    else if (mode == GRAD_POOL) go(k_grad_sum<GRAD_POOL>);
+    else go(k_grad_sum<GRAD_X>);
     return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 

@@ -49,7 +49,7 @@ def load():
         "nn_conv_dx": [vp, i32, i32, i32, i32, i32, vp, vp, vp],
         "nn_conv_dw": [vp, vp, i32, vp, i32, i32, i32, i32, i32, i32, i32, vp, vp],
         "nn_weight_t": [vp, i32, vp, vp, vp, vp, vp, vp, vp],
-        "nn_grad_sum": [vp, vp, i64, i32, i32, vp, vp, vp],
+        "nn_grad_sum": [vp, vp, i32, i32, i32, i32, vp, i32, i32, vp, vp, vp],
     }
     for name, args in sig.items():
         fn = getattr(lib, name)
@@ -79,6 +79,8 @@ def gemm(M, N, R, A, lda, ta, B, ldb, tb, Cm, ldc, bias=None, flags=0, splits=1)
 
 # input of a convolution: x, x upsampled x2, x + skip
 IN_X, IN_UP, IN_ADD = 0, 1, 2
+# gradient of an output: dy, dy through an upsampling, dy through a pooling + skip
+GRAD_X, GRAD_UP, GRAD_POOL = 0, 1, 2
 
 
 def conv(x, skip, mode, Bn, H, W, cin, cout, k, w, kp, bias, relu, y):
@@ -103,8 +105,11 @@ def weight_t(w, layers, wt):
     _check(load().nn_weight_t(_p(w), n, f, t, ci, co, kp, _p(wt), _stream()), "nn_weight_t")
 
 
-def grad_sum(dy, y, relu, N, dz, db):
-    _check(load().nn_grad_sum(_p(dy), _p(y), dy.numel(), int(relu), N, _p(dz), _p(db), _stream()), "nn_grad_sum")
+def grad_sum(dy, y, relu, N, dz, db, mode=GRAD_X, skip=None, dims=None):
+    """dims: (images, height, width) of the gradient that dy, mode and skip describe."""
+    Bn, H, W = dims or (1 if dy.numel() % N == 0 else -1, 1, max(1, dy.numel() // N))
+    _check(load().nn_grad_sum(_p(dy), _p(skip), mode, Bn, H, W, _p(y), int(relu), N, _p(dz), _p(db), _stream()),
+           "nn_grad_sum")
 
 
 def im2col(x, Bn, H, W, Cc, Kp, col):

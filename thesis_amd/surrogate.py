@@ -152,7 +152,11 @@ class Net:
         cache[li] = (x, skip, mode, y, Bn, H, W)
         return y
 
-    def _conv_bwd(self, dy, li, cache, need_dx=True):
+    def _conv_bwd(self, dy, li, cache, need_dx=True, mode_dy=nn.GRAD_X, skip_dy=None):
+        """Layer li's parameter gradients and, with need_dx, its input gradient,
+        from its output gradient: dy, or what mode_dy makes of it (GRAD_UP: dy
+        through the upsampling above; GRAD_POOL: dy through the pooling above,
+        plus skip_dy)."""
         _, cin, cout, k, relu = ARCH[li]
         kp = kpad(cin, k)
         x, skip, mode, y, Bn, H, W = cache[li]
@@ -160,7 +164,7 @@ class Net:
         wo, bo = self.wo[li], self.bo[li]
         dz = torch.empty(M * cout, dtype=torch.int16, device=self.dev)
         if cout % 32 == 0:
-            nn.grad_sum(dy, y, relu, cout, dz, self.g[bo:bo + cout])
+            nn.grad_sum(dy, y, relu, cout, dz, self.g[bo:bo + cout], mode_dy, skip_dy, (Bn, H, W))
         else:
             nn.grad_bf16(dy, y, relu, dz)
             nn.colsum(dy, y, relu, M, cout, self.g[bo:bo + cout])
@@ -224,7 +228,7 @@ class Net:
         is dout into self.g (zero it first)."""
         I = INDEX
         Bn, H, W = c["dims"]
-        H2, W2, H3, W3, H4, W4 = H // 2, W // 2, H // 4, W // 4, H // 8, W // 8
+        H4, W4 = H // 8, W // 8
         # transposed weights of the 3x3 layers whose input gradient is taken
         at, layers, off = {}, [], 0
         for li, (name, cin, cout, k, _) in enumerate(ARCH):
@@ -239,38 +243,23 @@ class Net:
         d = self._conv_bwd(d, I["d1b"], c)            # gradient of relu(d1a) + s1
         ds1 = d
         d = self._conv_bwd(d, I["d1a"], c)
-        da = self._new(Bn * H2 * W2 * 64)
-        nn.up2_bwd(d, Bn, H2, W2, 64, da)
-        d = self._conv_bwd(da, I["d2b"], c)
+        d = self._conv_bwd(d, I["d2b"], c, mode_dy=nn.GRAD_UP)
         ds2 = d
         d = self._conv_bwd(d, I["d2a"], c)
-        da = self._new(Bn * H3 * W3 * 128)
-        nn.up2_bwd(d, Bn, H3, W3, 128, da)
-        d = self._conv_bwd(da, I["d3b"], c)
+        d = self._conv_bwd(d, I["d3b"], c, mode_dy=nn.GRAD_UP)
         ds3 = d
         d = self._conv_bwd(d, I["d3a"], c)
-        da = self._new(Bn * H4 * W4 * 128)
-        nn.up2_bwd(d, Bn, H4, W4, 128, da)
-        d = self._conv_bwd(da, I["b2"], c)
+        d = self._conv_bwd(d, I["b2"], c, mode_dy=nn.GRAD_UP)
         dym = self._new(d.numel())
         nn.ymix(d, Bn, H4, W4, 128, dym)
         dxi = self._new(d.numel())
         nn.xint(dym, Bn, H4, W4, 128, 1, dxi)
         d = self._conv_bwd(dxi, I["b1"], c)
-        dp = self._new(Bn * H3 * W3 * 128)
-        nn.avgpool2_bwd(d, Bn, H3, W3, 128, dp)
-        nn.axpy(1.0, ds3, dp)
-        d = self._conv_bwd(dp, I["e3b"], c)
+        d = self._conv_bwd(d, I["e3b"], c, mode_dy=nn.GRAD_POOL, skip_dy=ds3)
         d = self._conv_bwd(d, I["e3a"], c)
-        dp = self._new(Bn * H2 * W2 * 64)
-        nn.avgpool2_bwd(d, Bn, H2, W2, 64, dp)
-        nn.axpy(1.0, ds2, dp)
-        d = self._conv_bwd(dp, I["e2b"], c)
+        d = self._conv_bwd(d, I["e2b"], c, mode_dy=nn.GRAD_POOL, skip_dy=ds2)
         d = self._conv_bwd(d, I["e2a"], c)
-        dp = self._new(Bn * H * W * 32)
-        nn.avgpool2_bwd(d, Bn, H, W, 32, dp)
-        nn.axpy(1.0, ds1, dp)
-        d = self._conv_bwd(dp, I["e1b"], c)
+        d = self._conv_bwd(d, I["e1b"], c, mode_dy=nn.GRAD_POOL, skip_dy=ds1)
         self._conv_bwd(d, I["e1a"], c, need_dx=False)
 
     def loss_grad(self, out, target, mask, wch):
