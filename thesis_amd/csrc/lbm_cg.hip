@@ -140,38 +140,20 @@ __device__ inline void cg_collide(const CgParams& cp, const T* h, const T* r, T 
     mac[0] = rr; mac[1] = rb; mac[2] = rho; mac[3] = u; mac[4] = v;
 }
 
-template <int H>
-__device__ inline void gradient(const float* __restrict__ psi, int lx, int ly, float& gx, float& gy) {
-    // psi tile row length TX + 2H, node (lx, ly) of the interior at (lx+H, ly+H)
-    constexpr int RW = TX + 2 * H;
-    float ax = 0, ay = 0;
+// Gradient at element `at` of an LDS field with rows of RW.
+template <int H, int RW, class T>
+__device__ inline void gradient(const T* __restrict__ psi, int at, T& gx, T& gy) {
+    T ax = 0, ay = 0;
 #pragma unroll
     for (int dy = -H; dy <= H; ++dy)
 #pragma unroll
         for (int dx = -H; dx <= H; ++dx) {
             const int c2 = dx * dx + dy * dy;
             if (c2 == 0) continue;
-            const float wk = H == 1 ? (c2 == 1 ? 4.0f / 12.0f : 1.0f / 12.0f) : (float)HOW(c2);
-            const float p = psi[(ly + H + dy) * RW + (lx + H + dx)];
-            if (dx) ax += wk * (float)dx * p;
-            if (dy) ay += wk * (float)dy * p;
-        }
-    gx = ax; gy = ay;
-}
-template <int H>
-__device__ inline void gradient(const double* __restrict__ psi, int lx, int ly, double& gx, double& gy) {
-    constexpr int RW = TX + 2 * H;
-    double ax = 0, ay = 0;
-#pragma unroll
-    for (int dy = -H; dy <= H; ++dy)
-#pragma unroll
-        for (int dx = -H; dx <= H; ++dx) {
-            const int c2 = dx * dx + dy * dy;
-            if (c2 == 0) continue;
-            const double wk = H == 1 ? (c2 == 1 ? 4.0 / 12.0 : 1.0 / 12.0) : HOW(c2);
-            const double p = psi[(ly + H + dy) * RW + (lx + H + dx)];
-            if (dx) ax += wk * (double)dx * p;
-            if (dy) ay += wk * (double)dy * p;
+            const T wk = (T)(H == 1 ? (c2 == 1 ? 4.0 / 12.0 : 1.0 / 12.0) : HOW(c2));
+            const T p = psi[at + dy * RW + dx];
+            if (dx) ax += wk * (T)dx * p;
+            if (dy) ay += wk * (T)dy * p;
         }
     gx = ax; gy = ay;
 }
@@ -232,8 +214,9 @@ __global__ __launch_bounds__(THREADS) void k_cg_step(const typename CIo<S>::raw*
         if (!inside[k]) continue;
         const int lx = tx, ly = ty + 8 * k, x = x0 + lx, y = y0 + ly;
         T gx, gy, dx = 0, dy = 0;
-        gradient<H>(psi, lx, ly, gx, gy);
-        if (E) gradient<H>(rt, lx, ly, dx, dy);
+        const int at = (ly + H) * RW + lx + H;
+        gradient<H, RW>(psi, at, gx, gy);
+        if (E) gradient<H, RW>(rt, at, dx, dy);
         T ho[9], ro[9], m[5];
         cg_collide<T, E>(cp, h[k], r[k], gx, gy, dx, dy, ho, ro, m);
         const uint32_t idx = (uint32_t)y * (uint32_t)nx + (uint32_t)x;
@@ -245,6 +228,83 @@ __global__ __launch_bounds__(THREADS) void k_cg_step(const typename CIo<S>::raw*
         if (write_macros) {
             const size_t n = (size_t)nx * ny;
             for (int a = 0; a < 5; ++a) mac[a * n + idx] = (double)m[a];
+        }
+    }
+}
+
+// Several steps per launch, FP64 and FP32 storage.  A workgroup takes a square of
+// 32 x 32 nodes, one a thread, pulls their populations once, advances them `steps`
+// steps with the moving links changing hands in LDS and stores the inner nodes.  The
+// pull makes every node's streamed state exact; a collision then costs H rings (the
+// gradient) and each further streaming one more, so a frame of `halo` >=
+// steps (1 + H) - 1 nodes is recomputed by the neighbouring squares.  The node update
+// is k_cg_step's on the same values: the results are its bits.  FP16 storage stays
+// with k_cg_step: there the conversion of a pulled value is fused into the density's
+// sum, and without that a rounding of 2^-11 falls the other way now and then.
+//
+// Per step, one launch a step / several (the number): FP64 64 x 64 7.3 / 3.6 us (6),
+// 250 x 187 8.1 / 4.5 (5), 512 x 512 17.6 / 15.2 (2), 1024 x 1024 69 / 52 (3); FP32
+// 5.8 / 2.8, 6.6 / 3.6, 10.3 / 8.4, 42 / 25; 24-point stencil FP64 250 x 187 8.5 / 5.5
+// (3), 1024 x 1024 76 / 66 (2).  What bounds it: on few squares the launch and the
+// chain of one node update a step (2.6 us FP64, seven divisions and a root), on many
+// the instructions, 1.5 times with the frame of two steps.
+// FULL: more squares than CUs; FP32 then keeps to 64 registers so that two
+// workgroups share a CU.
+constexpr int SIDE = 32, SQ = SIDE * SIDE;
+template <int S, int H, bool E, bool FULL>
+__global__ __launch_bounds__(SQ, S == 1 && FULL ? 8 : 4) void k_cg_multi(const typename CIo<S>::raw* __restrict__ src,
+                                                                       typename CIo<S>::raw* __restrict__ dst,
+                                                                       CgParams cp, int steps, int halo, uint32_t tx) {
+    using T = typename CIo<S>::T;
+    __shared__ T ex[16][SQ];
+    __shared__ T psi[SQ];
+    __shared__ T rt[E ? SQ : 1];
+    const int tid = threadIdx.x, lx = tid & (SIDE - 1), ly = tid / SIDE;
+    const int in = SIDE - 2 * halo, nx = cp.nx, ny = cp.ny;
+    const int rim = min(min(lx, SIDE - 1 - lx), min(ly, SIDE - 1 - ly));
+    const uint32_t b = xcd_block(blockIdx.x, gridDim.x, cp.xcd_shift, cp.xchunk_shift), by = b / tx;
+    const int ux = (int)(b - by * tx) * in - halo + lx, uy = (int)by * in - halo + ly;
+    auto pwrap = [](int a, int n) { return a >= 0 && a < n ? a : ((a % n) + n) % n; };
+    T h[9], r[9];
+    auto put = [&] {
+        T rho, rr;
+        densities<T>(h, r, rho, rr);
+        psi[tid] = ((T)2 * rr - rho) / rho;
+        if (E) rt[tid] = rho;
+    };
+    pull<S>(src, cp, pwrap(ux, nx), pwrap(uy, ny), h, r);
+    put();
+    for (int s = 0;;) {
+        __syncthreads();
+        const bool on = rim >= s * (1 + H) + H;
+        if (on) {
+            T gx, gy, dx = 0, dy = 0, m[5];
+            gradient<H, SIDE>(psi, tid, gx, gy);
+            if (E) gradient<H, SIDE>(rt, tid, dx, dy);
+            cg_collide<T, E>(cp, h, r, gx, gy, dx, dy, h, r, m);
+        }
+        if (++s == steps) break;
+        if (on) {
+#pragma unroll
+            for (int i = 1; i < 9; ++i) { ex[i - 1][tid] = h[i]; ex[7 + i][tid] = r[i]; }
+        }
+        __syncthreads();
+        if (rim >= s * (1 + H)) {   // at least one ring inside: every source is in the square
+#pragma unroll
+            for (int i = 1; i < 9; ++i) {
+                const int j = tid - CX[i] - SIDE * CY[i];
+                h[i] = ex[i - 1][j];
+                r[i] = ex[7 + i][j];
+            }
+            put();
+        }
+    }
+    if (rim >= halo && ux < nx && uy < ny) {   // ux, uy >= 0 inside the frame
+        const uint32_t idx = (uint32_t)uy * (uint32_t)nx + (uint32_t)ux;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            CIo<S>::st(dst, (uint32_t)i * cp.plane + idx, h[i], i, false);
+            CIo<S>::st(dst, (uint32_t)(9 + i) * cp.plane + idx, r[i], i, true);
         }
     }
 }
@@ -390,6 +450,26 @@ hipError_t cg_launch_step(int storage, int ho, const void* src, void* dst, const
     else { if (ho) CG_STEP_E(2, 2); else CG_STEP_E(2, 1); }
 #undef CG_STEP_E
 #undef CG_STEP
+    return hipGetLastError();
+}
+
+hipError_t cg_launch_multi(int storage, int ho, const void* src, void* dst, const cg::CgParams& cp, int steps, int most,
+                           hipStream_t st) {
+    const int halo = most * (ho ? 3 : 2) - 1, in = cg::SIDE - 2 * halo;
+    if (steps < 1 || steps > most || in < 1 || storage < 0 || storage > 1) return hipErrorInvalidValue;
+    const uint32_t tx = (uint32_t)(cp.nx + in - 1) / in, ty = (uint32_t)(cp.ny + in - 1) / in;
+#define CG_M(S_, H_, E_, F_)                                                                                 \
+    hipLaunchKernelGGL((cg::k_cg_multi<S_, H_, E_, F_>), dim3(tx * ty), dim3(cg::SQ), 0, st,                 \
+                       (const typename cg::CIo<S_>::raw*)src, (typename cg::CIo<S_>::raw*)dst, cp, steps, halo, tx)
+#define CG_M_E(S_, H_, F_) do { if (cp.enhanced) CG_M(S_, H_, true, F_); else CG_M(S_, H_, false, F_); } while (0)
+#define CG_M_H(S_, F_) do { if (ho) CG_M_E(S_, 2, F_); else CG_M_E(S_, 1, F_); } while (0)
+    const bool full = tx * ty > 256;
+    if (storage == 0) CG_M_H(0, false);
+    else if (full) CG_M_H(1, true);
+    else CG_M_H(1, false);
+#undef CG_M_H
+#undef CG_M_E
+#undef CG_M
     return hipGetLastError();
 }
 
