@@ -69,18 +69,18 @@ __device__ inline void pull(const typename CIo<S>::raw* __restrict__ src, const 
         r[i] = CIo<S>::ld(src, (uint32_t)(19 + i) * cp.plane + k, i, true);
     }
 }
-// The FP64 two-launch step's pull: each plane the scalar base of its load and
-// one 32-bit byte offset per link for both colours (k_cg3_psi: 100 -> 62
+// The FP64 and FP32 two-launch step's pull: each plane the scalar base of its load
+// and one 32-bit byte offset per link for both colours (k_cg3_psi FP64: 100 -> 62
 // registers); red(i, r_i) receives the red populations when R.
-template <bool R, class Red>
-__device__ inline void pull64(const double* __restrict__ src, const CgParams& cp, int x, int y, int z, double* h,
-                              Red red) {
+template <bool R, class T, class Red>
+__device__ inline void pull_raw(const T* __restrict__ src, const CgParams& cp, int x, int y, int z, T* h, Red red) {
 #pragma unroll
     for (int i = 0; i < 19; ++i) {
         const int sx = wrap(x - CX[i], cp.nx), sy = wrap(y - CY[i], cp.ny), sz = wrap(z - CZ[i], cp.nz);
-        const uint32_t k = (((uint32_t)sz * (uint32_t)cp.ny + (uint32_t)sy) * (uint32_t)cp.nx + (uint32_t)sx) * 8u;
-        h[i] = *(const double*)((const char*)(src + (uint32_t)i * cp.plane) + k);
-        if (R) red(i, *(const double*)((const char*)(src + (uint32_t)(19 + i) * cp.plane) + k));
+        const uint32_t k = (((uint32_t)sz * (uint32_t)cp.ny + (uint32_t)sy) * (uint32_t)cp.nx + (uint32_t)sx) *
+                           (uint32_t)sizeof(T);
+        h[i] = *(const T*)((const char*)(src + (uint32_t)i * cp.plane) + k);
+        if (R) red(i, *(const T*)((const char*)(src + (uint32_t)(19 + i) * cp.plane) + k));
     }
 }
 
@@ -262,10 +262,12 @@ __device__ inline bool node_of(const CgParams& cp, int& x, int& y, int& z) {
 }
 
 // Phase field of the post-streaming state (and with E its density in the
-// second N of psi).  FP64 storage keeps the red density too, in the third N: the
-// collision needs the red populations only through their sum, so the step then
-// pulls the deviations alone.  Not so in FP32 and FP16, where it measured no
-// gain (100 x 90 x 80: 71 us both ways).
+// second N of psi).  FP64 and FP32 storage keep the red density too, in the third N:
+// the collision needs the red populations only through their sum, so the step then
+// pulls the deviations alone (FP32 per step, both launches: 128^3 104-point 198 to
+// 179 us, 256^3 1483 to 1346, 192 x 96 x 61 18-point 90 to 77, 64 x 96 x 160 76 to 67).
+// Not so in FP16, whose step sums the rounded products of its conversion.  Bound by
+// memory: 4 of 6 values a link move now.
 template <int S, bool E>
 __global__ __launch_bounds__(BX * BY) void k_cg3_psi(const typename CIo<S>::raw* __restrict__ src, CgParams cp,
                                                      typename CIo<S>::T* __restrict__ psi) {
@@ -273,14 +275,14 @@ __global__ __launch_bounds__(BX * BY) void k_cg3_psi(const typename CIo<S>::raw*
     int x, y, z;
     if (!node_of(cp, x, y, z)) return;
     T h[19], r[19], rho, rr;
-    if constexpr (S == 0) pull64<true>(src, cp, x, y, z, h, [&](int i, double v) { r[i] = v; });
+    if constexpr (S < 2) pull_raw<true>(src, cp, x, y, z, h, [&](int i, T v) { r[i] = v; });
     else pull<S>(src, cp, x, y, z, h, r);
     densities<T>(h, r, rho, rr);
     const size_t n = (size_t)cp.nx * cp.ny * cp.nz;
     const uint32_t j = ((uint32_t)z * (uint32_t)cp.ny + (uint32_t)y) * (uint32_t)cp.nx + (uint32_t)x;
     psi[j] = ((T)2 * rr - rho) / rho;
     if (E) psi[n + j] = rho;
-    if (S == 0) psi[2 * n + j] = rr;
+    if (S < 2) psi[2 * n + j] = rr;
 }
 
 // FP32 and FP16 storage (FP64: k_cg3_step64)
@@ -292,8 +294,16 @@ __global__ __launch_bounds__(BX * BY) void k_cg3_step(const typename CIo<S>::raw
     using T = typename CIo<S>::T;
     int x, y, z;
     if (!node_of(cp, x, y, z)) return;
+    const uint32_t idx = ((uint32_t)z * (uint32_t)cp.ny + (uint32_t)y) * (uint32_t)cp.nx + (uint32_t)x;
     T h[19], r[19];
-    pull<S>(src, cp, x, y, z, h, r);
+    if constexpr (S < 2) {   // red populations that sum to the red density: x + (-0.0) is x
+        pull_raw<false>(src, cp, x, y, z, h, [](int, T) {});
+        r[0] = psi[2 * (size_t)cp.nx * cp.ny * cp.nz + idx];
+#pragma unroll
+        for (int i = 1; i < 19; ++i) r[i] = (T)-0.0;
+    } else {
+        pull<S>(src, cp, x, y, z, h, r);
+    }
     T gx, gy, gz, d[3] = {0, 0, 0};
     gradient<H, T, (S >= 2)>(cp, x, y, z, [psi](uint32_t j) { return psi[j]; }, gx, gy, gz);
     if (E) {
@@ -302,7 +312,6 @@ __global__ __launch_bounds__(BX * BY) void k_cg3_step(const typename CIo<S>::raw
     }
     T ho[19], ro[19], m[6];
     collide<T, E>(cp, h, r, gx, gy, gz, d, ho, ro, m);
-    const uint32_t idx = ((uint32_t)z * (uint32_t)cp.ny + (uint32_t)y) * (uint32_t)cp.nx + (uint32_t)x;
 #pragma unroll
     for (int i = 0; i < 19; ++i) {
         CIo<S>::st(dst, (uint32_t)i * cp.plane + idx, ho[i], i, false);
@@ -335,7 +344,7 @@ __global__ __launch_bounds__(BX * BY) void k_cg3_step64(const double* __restrict
     const uint32_t idx = ((uint32_t)z * (uint32_t)cp.ny + (uint32_t)y) * (uint32_t)cp.nx + (uint32_t)x;
     // red populations that sum to the red density: x + (-0.0) is x
     double h[19], r[19];
-    pull64<false>(src, cp, x, y, z, h, [](int, double) {});
+    pull_raw<false>(src, cp, x, y, z, h, [](int, double) {});
     r[0] = psi[2 * n + idx];
 #pragma unroll
     for (int i = 1; i < 19; ++i) r[i] = -0.0;

@@ -61,10 +61,11 @@ lbm_status cfail(lbm_cg_ctx* c, lbm_status s, const char* fmt, ...) {
     } while (0)
 // Column height of the single-pass D3Q19 step; 0: the two-launch step.
 //
-// Below 2^20 nodes, where the populations stay in the caches, two launches are
-// faster with FP64 and FP32 storage (FP32 per step: 64^3 21 / 23 us, 128 x 96 x 64
-// 59 / 68 us, 128 x 128 x 64 89 / 84 us); the two give the same bits there, not
-// with FP16, which keeps the single pass.
+// While the populations stay in the caches two launches are faster with FP64 and
+// FP32 storage, below 2^20 and 7/4 2^20 nodes (per step, single pass / two launches:
+// FP32 64^3 23 / 21 us, 192 x 96 x 61 92 / 77, 128 x 128 x 96 127 / 112, 128^3 158 /
+// 172; FP64 192 x 96 x 61 170 / 168, 128 x 128 x 96 218 / 233); the two give the same
+// bits there, not with FP16, which keeps the single pass.
 //
 // One workgroup of 64 x 8 nodes
 // fits a CU (139-254 registers), and a column costs its planes and two more for
@@ -74,7 +75,8 @@ lbm_status cfail(lbm_cg_ctx* c, lbm_status s, const char* fmt, ...) {
 // 95 us).  At most 32 planes (64 with FP16 storage): taller columns lose more
 // to the caches (256^3 FP32 1.153 ms at 32, 1.206 ms at 64).
 int cg3_zchunk(int nx, int ny, int nz, int rows, int storage) {
-    if (storage != LBM_STORE_F16 && (size_t)nx * ny * nz < (size_t)1 << 20) return 0;
+    const size_t n = (size_t)nx * ny * nz;
+    if ((storage == LBM_STORE_F64 && n < (size_t)4 << 18) || (storage == LBM_STORE_F32 && n < (size_t)7 << 18)) return 0;
     const long tiles = (long)(nx / 64) * (ny / rows), cus = 256;
     const int most = storage == LBM_STORE_F16 ? 64 : 32;
     int best = most;
