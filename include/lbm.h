@@ -270,7 +270,7 @@ const char* lbm_latticegen_last_error(void);
  * (S/GpuUpdateMacro.cu:215-361) and the sums of S/Iterate3D.cu:637-645,
  * driven by S/Iterate3D.cu:495-800.  Colour parameters as in S/main.cu:52-72.
  * A box with walls or a body force runs the reference's order instead
- * (collide, stream, wall condition, macros; two launches per step). */
+ * (collide, stream, wall condition, macros; two launches per step, one for D2Q9 FP64). */
 typedef struct lbm_cg_ctx lbm_cg_ctx;
 typedef struct {
     uint32_t abi_version;
