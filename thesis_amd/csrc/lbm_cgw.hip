@@ -252,6 +252,14 @@ __device__ inline double wall_row64(double (&f)[9], int walls, double u, double 
     return r;
 }
 
+// a / b from ib = 1 / b: the product and one correction, good to the last bit.  The
+// plain product gave colour shares that add to the same side of 1 at a node every
+// step, and so a drift of its mass.
+__device__ inline double quot(double a, double b, double ib) {
+    const double q = a * ib;
+    return fma(fma(-q, b, a), ib, q);
+}
+
 // One FP64 step in a single launch, populations and macros from one pair of
 // buffers to the other.
 //
@@ -359,7 +367,7 @@ __global__ __launch_bounds__(BX * BY) void k_cgw_step64(const double* __restrict
                 }
         }
     }
-    const double kr = rr * ir, kb = br * ir, kk = cp.beta * rr * kb;
+    const double kr = quot(rr, r, ir), kb = quot(br, r, ir), kk = cp.beta * rr * kb;
     const double mean_nu = (cp.r_nu * cp.b_nu) / (kr * cp.b_nu + kb * cp.r_nu);
     double iom = 3.0 * mean_nu + 0.5;
     const double om = 1.0 / iom, alpha = cp.r_alpha * kr + cp.b_alpha * kb;
@@ -424,8 +432,8 @@ __global__ __launch_bounds__(BX * BY) void k_cgw_step64(const double* __restrict
     macn[ind] = R;
     macn[n + ind] = B;
     macn[2 * n + ind] = rn;
-    macn[3 * n + ind] = jx * irn + (wp.external_force ? gs * irn : 0.0);
-    macn[4 * n + ind] = jy * irn + (wp.external_force ? 0.0 : gs);
+    macn[3 * n + ind] = quot(jx, rn, irn) + (wp.external_force ? gs * irn : 0.0);
+    macn[4 * n + ind] = quot(jy, rn, irn) + (wp.external_force ? 0.0 : gs);
 }
 
 // Rest-state colours from colour densities (S/GpuInit.cu:323-352), or given
