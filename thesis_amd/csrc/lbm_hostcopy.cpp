@@ -69,6 +69,21 @@ hipError_t plain(const OutCopy* c, int n, hipStream_t st) {
     return hipStreamSynchronize(st);
 }
 
+// Makes dev the calling thread's current device while it lives: a stream's events
+// have to be of its device, and the caller's device is not this file's to change.
+struct OnDevice {
+    int was = -1;
+    hipError_t e;
+    explicit OnDevice(int dev) {
+        int now = dev;
+        e = hipGetDevice(&now);
+        if (e == hipSuccess && now != dev && (e = hipSetDevice(dev)) == hipSuccess) was = now;
+    }
+    ~OnDevice() {
+        if (was >= 0) (void)hipSetDevice(was);
+    }
+};
+
 struct Piece {
     char* dst;
     const char* src;
@@ -111,10 +126,11 @@ hipError_t copy_to_host(const OutCopy* c, int n, int dev, hipStream_t st) {
                                             (size_t)std::max(1u, std::thread::hardware_concurrency())});
     if (want < 2) return plain(c, n, st);
     try {
+        const OnDevice on(dev);
         std::vector<void*> buf = take(2 * want, total >= kMakeFrom);
         const int nt = (int)buf.size() / 2;
         hipEvent_t ev[2 * kMaxThreads] = {};
-        hipError_t e = hipSuccess;
+        hipError_t e = on.e;
         for (int i = 0; i < 2 * nt && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
         bool done = false;
         if (nt >= 2 && e == hipSuccess) {
@@ -123,8 +139,9 @@ hipError_t copy_to_host(const OutCopy* c, int n, int dev, hipStream_t st) {
                 for (size_t o = 0; o < c[i].bytes; o += kChunk)
                     p.push_back({(char*)c[i].dst + o, (const char*)c[i].src + o, std::min(kChunk, c[i].bytes - o)});
             std::atomic<int> err{(int)hipSuccess};
-            auto work = [&](int t) {
-                hipError_t r = hipSetDevice(dev);
+            auto work = [&](int t) {   // on the caller's thread and on new ones
+                const OnDevice mine(dev);
+                hipError_t r = mine.e;
                 if (r == hipSuccess) r = drain(p, (size_t)t, (size_t)nt, &buf[2 * t], &ev[2 * t], st);
                 if (r != hipSuccess) err = (int)r;
             };
