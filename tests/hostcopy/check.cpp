@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -14,12 +15,21 @@ thread_local hipError_t t_last = hipSuccess;
 thread_local int t_dev = 0;
 std::atomic<int> events{0}, buffers{0}, direct{0}, staged{0};
 std::atomic<int> buffers_allowed{1 << 20}, events_allowed{1 << 20};
+std::atomic<int> news_allowed{1 << 30};   // the next allocations by new; then one throws
 
 hipError_t res(hipError_t e) {
     if (e != hipSuccess) t_last = e;
     return e;
 }
 }  // namespace
+
+void* operator new(size_t n) {
+    if (news_allowed-- == 0) throw std::bad_alloc();
+    if (void* p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 hipError_t hipGetLastError() {
     const hipError_t e = t_last;
@@ -77,6 +87,26 @@ void device() {
     want(t_dev == 0, "the caller's current device is what it was");
     want((staged > 0 && direct == 0) || std::thread::hardware_concurrency() < 2, "it went through the staging buffers");
 }
+
+// Host memory that runs out at every allocation of the copy in turn: the fields
+// arrive, and the next copy has the buffers it had before.
+void memory() {
+    want(copy(0), "the first copy succeeds");
+    const int made = buffers;
+    for (int k = 0; k < 200; ++k) {
+        news_allowed = k;
+        want(copy(0), "a copy without memory succeeds");
+        const bool thrown = news_allowed < 0;
+        news_allowed = 1 << 30;
+        want(events == 0, "its events are destroyed");
+        buffers_allowed = 0;   // what is idle has to do
+        staged = direct = 0;
+        want(copy(0) && (direct == 0 || made == 0), "its buffers are there for the next copy");
+        buffers_allowed = 1 << 20;
+        if (!thrown || bad) break;
+    }
+    want(buffers == made, "no buffer is made again");
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -84,6 +114,7 @@ int main(int argc, char** argv) {
     lbm::host_staging_retain();
     const char* name = argc > 1 ? argv[1] : "";
     if (!std::strcmp(name, "device")) device();
+    else if (!std::strcmp(name, "memory")) memory();
     else want(false, "a case of that name");
     want(events == 0, "every event is destroyed");
     lbm::host_staging_release();

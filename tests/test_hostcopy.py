@@ -25,3 +25,7 @@ def holds(r):
 
 def test_context_of_another_device(check):
     holds(check("device"))
+
+
+def test_host_memory_runs_out(check):
+    holds(check("memory"))

@@ -26,40 +26,46 @@ constexpr size_t kPerThread = (size_t)2 << 20;
 constexpr size_t kMakeFrom = (size_t)24 << 20;
 
 std::mutex g_mutex;
-std::vector<void*> g_free;                   // idle staging buffers
-int g_made = 0, g_holders = 0;
-
-// Up to n staging buffers, idle ones and, when make is set, new ones (fewer when
-// others hold them).
-std::vector<void*> take(int n, bool make) {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    std::vector<void*> got;
-    got.reserve((size_t)n);
-    while ((int)got.size() < n) {
-        if (!g_free.empty()) {
-            got.push_back(g_free.back());
-            g_free.pop_back();
-            continue;
-        }
-        void* p = nullptr;
-        if (!make || g_made >= 2 * kMaxThreads || hipHostMalloc(&p, kChunk, hipHostMallocPortable) != hipSuccess) break;
-        ++g_made;
-        got.push_back(p);
-    }
-    return got;
-}
+void* g_free[2 * kMaxThreads];               // idle staging buffers
+int g_idle = 0, g_made = 0, g_holders = 0;
 
 void drop_idle() {   // g_mutex held
-    for (void* p : g_free) (void)hipHostFree(p);
-    g_made -= (int)g_free.size();
-    g_free.clear();
+    for (int i = 0; i < g_idle; ++i) (void)hipHostFree(g_free[i]);
+    g_made -= g_idle;
+    g_idle = 0;
 }
 
-void give(const std::vector<void*>& b) {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    g_free.insert(g_free.end(), b.begin(), b.end());
-    if (g_holders == 0) drop_idle();
-}
+// The buffers and events of one copy, given back on every way out; nothing here
+// allocates host memory.
+struct Staging {
+    void* buf[2 * kMaxThreads];
+    hipEvent_t ev[2 * kMaxThreads] = {};
+    int n = 0;   // buffers held
+    // Up to want buffers, idle ones and, when make is set, new ones (fewer when
+    // others hold them).
+    Staging(int want, bool make) {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        while (n < want) {
+            if (g_idle > 0) {
+                buf[n++] = g_free[--g_idle];
+                continue;
+            }
+            void* p = nullptr;
+            if (!make || g_made >= 2 * kMaxThreads || hipHostMalloc(&p, kChunk, hipHostMallocPortable) != hipSuccess) break;
+            ++g_made;
+            buf[n++] = p;
+        }
+    }
+    ~Staging() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+        std::lock_guard<std::mutex> lock(g_mutex);
+        for (int i = 0; i < n; ++i) g_free[g_idle++] = buf[i];
+        if (g_holders == 0) drop_idle();
+    }
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+};
 
 hipError_t plain(const OutCopy* c, int n, hipStream_t st) {
     for (int i = 0; i < n; ++i) {
@@ -117,6 +123,45 @@ hipError_t drain(const std::vector<Piece>& p, size_t t, size_t nt, void* const* 
     return e;
 }
 
+// The copies by up to `want` threads; false when nothing was started (no buffers,
+// events or host memory for them), else e is the outcome.
+bool staged(const OutCopy* c, int n, int dev, hipStream_t st, int want, bool make, hipError_t& e) {
+    try {
+        const OnDevice on(dev);
+        Staging s(2 * want, make);
+        const int nt = s.n / 2;
+        e = on.e;
+        for (int i = 0; i < 2 * nt && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&s.ev[i], hipEventDisableTiming);
+        if (nt < 2 || e != hipSuccess) return false;
+        std::vector<Piece> p;
+        for (int i = 0; i < n; ++i)
+            for (size_t o = 0; o < c[i].bytes; o += kChunk)
+                p.push_back({(char*)c[i].dst + o, (const char*)c[i].src + o, std::min(kChunk, c[i].bytes - o)});
+        std::atomic<int> err{(int)hipSuccess};
+        auto work = [&](int t) {   // on the caller's thread and on new ones
+            const OnDevice mine(dev);
+            hipError_t r = mine.e;
+            if (r == hipSuccess) r = drain(p, (size_t)t, (size_t)nt, &s.buf[2 * t], &s.ev[2 * t], st);
+            if (r != hipSuccess) err = (int)r;
+        };
+        std::vector<std::thread> th;
+        th.reserve((size_t)nt);
+        int started = 1;
+        try {
+            for (; started < nt; ++started) th.emplace_back(work, started);
+        } catch (...) {   // no more threads: this one takes their shares
+        }
+        work(0);
+        for (int t = started; t < nt; ++t) work(t);
+        for (auto& t : th) t.join();
+        e = (hipError_t)err.load();
+        if (e != hipSuccess) (void)hipStreamSynchronize(st);   // nothing in flight into the buffers
+        return true;
+    } catch (...) {
+        return false;
+    }
+}
+
 }  // namespace
 
 hipError_t copy_to_host(const OutCopy* c, int n, int dev, hipStream_t st) {
@@ -124,48 +169,9 @@ hipError_t copy_to_host(const OutCopy* c, int n, int dev, hipStream_t st) {
     for (int i = 0; i < n; ++i) total += c[i].bytes;
     const int want = (int)std::min<size_t>({(size_t)kMaxThreads, total / kPerThread,
                                             (size_t)std::max(1u, std::thread::hardware_concurrency())});
-    if (want < 2) return plain(c, n, st);
-    try {
-        const OnDevice on(dev);
-        std::vector<void*> buf = take(2 * want, total >= kMakeFrom);
-        const int nt = (int)buf.size() / 2;
-        hipEvent_t ev[2 * kMaxThreads] = {};
-        hipError_t e = on.e;
-        for (int i = 0; i < 2 * nt && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
-        bool done = false;
-        if (nt >= 2 && e == hipSuccess) {
-            std::vector<Piece> p;
-            for (int i = 0; i < n; ++i)
-                for (size_t o = 0; o < c[i].bytes; o += kChunk)
-                    p.push_back({(char*)c[i].dst + o, (const char*)c[i].src + o, std::min(kChunk, c[i].bytes - o)});
-            std::atomic<int> err{(int)hipSuccess};
-            auto work = [&](int t) {   // on the caller's thread and on new ones
-                const OnDevice mine(dev);
-                hipError_t r = mine.e;
-                if (r == hipSuccess) r = drain(p, (size_t)t, (size_t)nt, &buf[2 * t], &ev[2 * t], st);
-                if (r != hipSuccess) err = (int)r;
-            };
-            std::vector<std::thread> th;
-            th.reserve((size_t)nt);
-            int started = 1;
-            try {
-                for (; started < nt; ++started) th.emplace_back(work, started);
-            } catch (...) {   // no more threads: this one takes their shares
-            }
-            work(0);
-            for (int t = started; t < nt; ++t) work(t);
-            for (auto& t : th) t.join();
-            e = (hipError_t)err.load();
-            done = true;
-        }
-        if (done && e != hipSuccess) (void)hipStreamSynchronize(st);   // nothing in flight into the buffers
-        for (int i = 0; i < 2 * nt; ++i)
-            if (ev[i]) (void)hipEventDestroy(ev[i]);
-        give(buf);
-        return done ? e : plain(c, n, st);
-    } catch (...) {
-        return plain(c, n, st);
-    }
+    hipError_t e = hipSuccess;
+    if (want >= 2 && staged(c, n, dev, st, want, total >= kMakeFrom, e)) return e;
+    return plain(c, n, st);
 }
 
 void host_staging_retain() {
