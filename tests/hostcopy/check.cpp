@@ -107,6 +107,21 @@ void memory() {
     }
     want(buffers == made, "no buffer is made again");
 }
+
+// What runs out and is done without leaves no error behind for the thread's next
+// launch to report.
+void errors() {
+    hipGetLastError();
+    buffers_allowed = 0;
+    want(copy(0), "a copy without pinned memory succeeds");
+    want(hipGetLastError() == hipSuccess, "and leaves no error");
+    buffers_allowed = 5;
+    want(copy(0), "a copy with a part of the pinned memory succeeds");
+    want(hipGetLastError() == hipSuccess, "and leaves no error");
+    events_allowed = 3;
+    want(copy(0), "a copy without events succeeds");
+    want(hipGetLastError() == hipSuccess, "and leaves no error");
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -115,6 +130,7 @@ int main(int argc, char** argv) {
     const char* name = argc > 1 ? argv[1] : "";
     if (!std::strcmp(name, "device")) device();
     else if (!std::strcmp(name, "memory")) memory();
+    else if (!std::strcmp(name, "errors")) errors();
     else want(false, "a case of that name");
     want(events == 0, "every event is destroyed");
     lbm::host_staging_release();

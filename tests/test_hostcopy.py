@@ -29,3 +29,7 @@ def test_context_of_another_device(check):
 
 def test_host_memory_runs_out(check):
     holds(check("memory"))
+
+
+def test_pinned_memory_and_events_run_out(check):
+    holds(check("errors"))

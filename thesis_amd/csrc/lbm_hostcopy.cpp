@@ -51,7 +51,11 @@ struct Staging {
                 continue;
             }
             void* p = nullptr;
-            if (!make || g_made >= 2 * kMaxThreads || hipHostMalloc(&p, kChunk, hipHostMallocPortable) != hipSuccess) break;
+            if (!make || g_made >= 2 * kMaxThreads) break;
+            if (hipHostMalloc(&p, kChunk, hipHostMallocPortable) != hipSuccess) {
+                (void)hipGetLastError();
+                break;
+            }
             ++g_made;
             buf[n++] = p;
         }
@@ -125,6 +129,9 @@ hipError_t drain(const std::vector<Piece>& p, size_t t, size_t nt, void* const* 
 
 // The copies by up to `want` threads; false when nothing was started (no buffers,
 // events or host memory for them), else e is the outcome.
+//
+// What fails here and is done without must not stay behind as the thread's last
+// error: the next launch would report it as its own.
 bool staged(const OutCopy* c, int n, int dev, hipStream_t st, int want, bool make, hipError_t& e) {
     try {
         const OnDevice on(dev);
@@ -132,6 +139,7 @@ bool staged(const OutCopy* c, int n, int dev, hipStream_t st, int want, bool mak
         const int nt = s.n / 2;
         e = on.e;
         for (int i = 0; i < 2 * nt && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&s.ev[i], hipEventDisableTiming);
+        if (e != hipSuccess) (void)hipGetLastError();
         if (nt < 2 || e != hipSuccess) return false;
         std::vector<Piece> p;
         for (int i = 0; i < n; ++i)
