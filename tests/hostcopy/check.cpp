@@ -15,6 +15,8 @@ thread_local hipError_t t_last = hipSuccess;
 thread_local int t_dev = 0;
 std::atomic<int> events{0}, buffers{0}, direct{0}, staged{0};
 std::atomic<int> buffers_allowed{1 << 20}, events_allowed{1 << 20};
+const void* pinned = nullptr;      // memory that the runtime knows
+bool refuses_unknown = false;      // whether asking for other memory's attributes is an error
 std::atomic<int> news_allowed{1 << 30};   // the next allocations by new; then one throws
 
 hipError_t res(hipError_t e) {
@@ -45,6 +47,10 @@ hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
     return hipSuccess;
 }
 hipError_t hipHostFree(void* p) { std::free(p); --buffers; return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+    a->type = p == pinned ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
+    return res(p != pinned && refuses_unknown ? hipErrorInvalidValue : hipSuccess);
+}
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
     if (events >= events_allowed) return res(hipErrorOutOfMemory);
     *e = (FakeEvent*)std::malloc(sizeof(FakeEvent));
@@ -122,6 +128,22 @@ void errors() {
     want(copy(0), "a copy without events succeeds");
     want(hipGetLastError() == hipSuccess, "and leaves no error");
 }
+
+// Pinned memory of the caller takes the card's own copy, other memory the staging
+// buffers, whichever way the runtime says that it does not know it.
+void own_pinned() {
+    pinned = dst.data();
+    want(copy(0), "a copy into pinned memory succeeds");
+    want(staged == 0 && direct == 1, "without the staging buffers");
+    pinned = nullptr;
+    for (bool refuses : {false, true}) {
+        refuses_unknown = refuses;
+        staged = direct = 0;
+        want(copy(0), "a copy into other memory succeeds");
+        want((staged > 0 && direct == 0) || std::thread::hardware_concurrency() < 2, "through the staging buffers");
+        want(hipGetLastError() == hipSuccess, "and leaves no error");
+    }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -131,6 +153,7 @@ int main(int argc, char** argv) {
     if (!std::strcmp(name, "device")) device();
     else if (!std::strcmp(name, "memory")) memory();
     else if (!std::strcmp(name, "errors")) errors();
+    else if (!std::strcmp(name, "pinned")) own_pinned();
     else want(false, "a case of that name");
     want(events == 0, "every event is destroyed");
     lbm::host_staging_release();

@@ -33,3 +33,7 @@ def test_host_memory_runs_out(check):
 
 def test_pinned_memory_and_events_run_out(check):
     holds(check("errors"))
+
+
+def test_pinned_destination(check):
+    holds(check("pinned"))

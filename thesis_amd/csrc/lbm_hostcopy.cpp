@@ -79,6 +79,16 @@ hipError_t plain(const OutCopy* c, int n, hipStream_t st) {
     return hipStreamSynchronize(st);
 }
 
+// Memory that the runtime knows (pinned by the caller): the card writes it itself,
+// which beats staging and copying again (256^3, 537 MB: 9.4 / 17.3 ms; 28 MB 0.54 /
+// 1.0 ms).
+bool known(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();   // some runtimes refuse the question for other memory
+    return false;
+}
+
 // Makes dev the calling thread's current device while it lives: a stream's events
 // have to be of its device, and the caller's device is not this file's to change.
 struct OnDevice {
@@ -178,7 +188,8 @@ hipError_t copy_to_host(const OutCopy* c, int n, int dev, hipStream_t st) {
     const int want = (int)std::min<size_t>({(size_t)kMaxThreads, total / kPerThread,
                                             (size_t)std::max(1u, std::thread::hardware_concurrency())});
     hipError_t e = hipSuccess;
-    if (want >= 2 && staged(c, n, dev, st, want, total >= kMakeFrom, e)) return e;
+    if (want >= 2 && std::none_of(c, c + n, [](const OutCopy& o) { return known(o.dst); }) &&
+        staged(c, n, dev, st, want, total >= kMakeFrom, e)) return e;
     return plain(c, n, st);
 }
 
