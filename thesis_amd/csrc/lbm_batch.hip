@@ -8,7 +8,8 @@
 // separates steps.  Between checks it advances `halo` steps a barrier instead, over
 // squares of 32 x 32 nodes held in LDS with a frame of `halo` recomputed nodes
 // (lbm_square.h); the check's own step is a single one, since it reads the state
-// before it.  64 channels, 3.65 M nodes, FP64: 133 us a step with a barrier each
+// before it; halo follows from the sizes and the check interval (lbm_plan.h), 1 for
+// none.  64 channels, 3.65 M nodes, FP64: 133 us a step with a barrier each
 // (3.9 TB/s), 63 us with four; what bounds it now: the node update's
 // instructions, 1.8 times with the frame.  Nodes are stored densely per instance, so the source of
 // every pulled population is the node index minus (cx + cy nx): no index maps

@@ -9,6 +9,7 @@
 #include "lbm.h"
 #include "lbm_batch_internal.h"
 #include "lbm_hostcopy.h"
+#include "lbm_plan.h"
 
 #include <hip/hip_runtime.h>
 
@@ -32,9 +33,9 @@ struct lbm_batch {
     std::vector<int64_t> steps;     // steps since its initialisation
     std::vector<int> par;           // host copy of the buffer holding each instance's newest state
     size_t ndense = 0, nslots = 0, nfluid = 0, maxn = 0;
-    int ntiles = 0, grid = 0;
+    int ntiles = 0, blocks = 0;   // blocks: most workgroups of a grid
     int dev = 0;                  // device current at creation
-    int halo = 1, nsquares = 0;   // several-step phases: steps a barrier, squares of all instances
+    int halo = 1;                 // steps a barrier that the instance table's squares are for (1: none)
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<void*> allocs;
@@ -191,33 +192,6 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
         if (dbase >= 0xFFFFFFFFull || pbase >= 0xFFFFFFFFull || tbase >= (size_t)INT_MAX)
             return reject("batch too large");
     }
-    // Steps a barrier between checks: a phase of t steps costs about 25 us for the
-    // barrier (0.1 us a workgroup) and 6 + 1.25 t us for each round of 248 squares
-    // of 32 - 2t nodes a side; the t with the least time a step (lbm_api.cpp has the
-    // same model for one lattice).
-    auto squares = [&](int t) {
-        const int side = 32 - 2 * t;
-        size_t s = 0;
-        for (const BInst& B : hinst) s += (size_t)((B.nx + side - 1) / side) * ((B.ny + side - 1) / side);
-        return s;
-    };
-    int halo = 1;
-    double cost = 0;
-    for (int t = 2; t <= 10; ++t) {
-        const double c = (25.0 + std::ceil((double)squares(t) / 248.0) * (6.0 + 1.25 * t)) / t;
-        if (halo == 1 || c < cost) { cost = c; halo = t; }
-    }
-    const size_t nsq = squares(halo);
-    if (nsq >= (size_t)INT_MAX) return reject("batch too large");
-    {
-        size_t at = 0;
-        const int side = 32 - 2 * halo;
-        for (BInst& B : hinst) {
-            B.mbase = (uint32_t)at;
-            B.mtx = (uint32_t)((B.nx + side - 1) / side);
-            at += (size_t)B.mtx * ((B.ny + side - 1) / side);
-        }
-    }
     const size_t raw = storage == LBM_STORE_F64 ? 8 : 4;
 
     int ndev = 0;
@@ -243,8 +217,6 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
     b->nfluid = nfluid;
     b->maxn = maxn;
     b->ntiles = (int)tbase;
-    b->halo = halo;
-    b->nsquares = (int)nsq;
     auto bad = [&](lbm_status s) {
         g_create_err = b->err;
         lbm_batch_destroy(b);
@@ -259,8 +231,7 @@ lbm_status lbm_batch_create(const lbm_batch_instance* in, int32_t n, int32_t col
     // workgroup per XCD of headroom below the occupancy query's co-residency,
     // so that a CU the runtime keeps back cannot leave the grid waiting
     const int head = maxb >= 64 ? 8 : (maxb > 1 ? 1 : 0);
-    const int most = std::max(b->ntiles, b->nsquares);
-    b->grid = most < maxb - head ? most : maxb - head;
+    b->blocks = maxb - head;
     if (hipStreamCreate(&b->stream) != hipSuccess || hipEventCreate(&b->ev0) != hipSuccess ||
         hipEventCreate(&b->ev1) != hipSuccess) {
         b->err = "stream or event creation failed";
@@ -352,11 +323,25 @@ lbm_status lbm_batch_run(lbm_batch* b, double tol, int32_t check_every, int64_t 
     BCHK(b, hipMemcpyAsync(b->bs.acc, dz.data(), sizeof(double) * 2 * n, h2d, b->stream));
     BCHK(b, hipMemcpyAsync(b->bs.res, rinf.data(), sizeof(double) * n, h2d, b->stream));
     BCHK(b, hipMemcpyAsync(b->bs.remaining, &remaining, sizeof(int), h2d, b->stream));
+    // the last step is a check too
+    const BatchPlan plan = batch_plan(b->hinst.data(), n, b->ntiles, b->blocks, std::min<int64_t>(check_every, max_steps));
+    if (plan.halo > 1 && plan.halo != b->halo) {
+        uint32_t at = 0;
+        const int side = 32 - 2 * plan.halo;
+        for (BInst& B : b->hinst) {
+            B.mbase = at;
+            B.mtx = (uint32_t)((B.nx + side - 1) / side);
+            at += (uint32_t)squares_of(B.nx, B.ny, side);
+        }
+        b->halo = 1;
+        BCHK(b, hipMemcpyAsync(b->inst, b->hinst.data(), sizeof(BInst) * n, h2d, b->stream));
+        b->halo = plan.halo;
+    }
     BCHK(b, hipEventRecord(b->ev0, b->stream));
     if (max_steps > 0)
         BCHK(b, batch_run(b->storage == LBM_STORE_F64 ? 0 : 1, b->collision, b->inst, n, b->ntiles, b->P[0],
                           b->P[1], b->nodew, bfields(b), b->up, b->vp, b->bs, tol, check_every, (int)max_steps,
-                          b->halo, b->nsquares, b->grid, b->stream));
+                          plan.halo, (int)plan.squares, plan.grid, b->stream));
     BCHK(b, hipEventRecord(b->ev1, b->stream));
     std::vector<int> done(n);
     std::vector<double> res(n);
