@@ -22,6 +22,12 @@ int main() {
             }
             const lbm::BatchPlan p = lbm::batch_plan(s.data(), n, tiles, 248, every);
             std::printf("%d %ld %d\n", p.halo, p.squares, p.grid);
+        } else if (!std::strcmp(what, "flow2")) {
+            int nx, ny, f64, mrt;
+            size_t nf;
+            if (std::scanf("%d %d %zu %d %d", &nx, &ny, &nf, &f64, &mrt) != 5) return 1;
+            const lbm::StepPlan p = lbm::flow2_plan(nx, ny, nf, f64 != 0, mrt != 0);
+            std::printf("%d %d\n", p.most, p.least);
         } else {
             return 1;
         }

@@ -7,6 +7,7 @@
 #include "lbm.h"
 #include "lbm_hostcopy.h"
 #include "lbm_internal.h"
+#include "lbm_plan.h"
 
 #include <hip/hip_runtime.h>
 
@@ -33,7 +34,7 @@ struct lbm_ctx {
     void* P[2] = {nullptr, nullptr};      // population buffers (256 B into their allocations)
     void* Palloc[2] = {nullptr, nullptr};
     int cur = 0;              // buffer holding the newest post-collision state
-    int multi = 1;            // D2Q9: most steps of one launch (1: one launch per step)
+    StepPlan plan{1, 2};      // D2Q9: steps of one launch
     int64_t steps = -1;       // steps since the state was set; -1: no state
     uint32_t* node = nullptr;
     uint32_t* cidx = nullptr;     // dense node -> compact population index (all ones: solid)
@@ -130,24 +131,6 @@ lbm_status ensure_fout(lbm_ctx* c) {
     return dalloc(c, (void**)&c->fout, sizeof(double) * c->n * c->q);
 }
 
-// Steps per launch of a D2Q9 lattice (lbm_multi2.hip): with t steps the squares
-// advance 32 - 2t nodes a side, a launch costs about 6 us and 1.25 us a step for
-// each round of 256 squares; the smallest (rounds) x (6 + 1.25 t) / t.  Measured
-// per step at t = 3, 4, 5, 8, 12 (FP64): 256 x 64 3.75, 3.30, 3.02, 2.41, 2.01 us
-// (12 chosen), 500 x 120 3.91, 3.34, 3.04, 2.58, 5.92 (8), 1021 x 256 7.11, 6.02,
-// 7.20, 8.54, 22.3 (4); one launch a step 5.73, 6.27, 10.7.
-int multi2_steps(int nx, int ny) {
-    int best = 1;
-    double cost = 0;
-    for (int t = 2; t <= 14; ++t) {
-        const int in = 32 - 2 * t;
-        const double squares = (double)((nx + in - 1) / in) * ((ny + in - 1) / in);
-        const double c = std::ceil(squares / 256.0) * (6.0 + 1.25 * t) / t;
-        if (best == 1 || c < cost) { cost = c; best = t; }
-    }
-    return best;
-}
-
 // macros_last: the last launch also writes the FP64 macroscopic fields
 // (timed runs leave them to an untimed moments pass, refresh_macros).
 // ev_after (optional, nsteps events): recorded after each launch.
@@ -156,10 +139,10 @@ int multi2_steps(int nx, int ny) {
 // before it, which the reconstructions need, from the other buffer.
 lbm_status run_steps(lbm_ctx* c, int64_t nsteps, bool macros_last = true, hipEvent_t* ev_after = nullptr) {
     int64_t k = 0;
-    while (c->multi > 1 && !ev_after && nsteps - 1 - k > 1) {
-        const int m = (int)std::min<int64_t>(c->multi, nsteps - 1 - k);
+    while (c->plan.most > 1 && !ev_after && nsteps - 1 - k >= c->plan.least) {
+        const int m = (int)std::min<int64_t>(c->plan.most, nsteps - 1 - k);
         hipError_t e = launch_multi2(c->p.storage, c->p.collision, c->kp, c->P[c->cur], c->P[c->cur ^ 1], c->node,
-                                     c->cidx, fields(c), m, c->multi, c->stream);
+                                     c->cidx, fields(c), m, c->plan.most, c->stream);
         if (e != hipSuccess) return fail(c, LBM_EDEVICE, "step launch: %s", hipGetErrorString(e));
         c->cur ^= 1;
         k += m;
@@ -586,10 +569,10 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
     k.rank = rank_fits ? 1 : 0;
     if (const char* e = std::getenv("LBM_RANK")) k.rank = rank_fits && e[0] == '1';
     if (p->q == 9 && p->storage <= LBM_STORE_F32 && k.rank && k.tile) {
-        c->multi = multi2_steps(p->nx, p->ny);   // LBM_MULTI: steps per launch, 1 for one each
-        if (const char* e = std::getenv("LBM_MULTI")) {
+        c->plan = flow2_plan(p->nx, p->ny, nf, p->storage == LBM_STORE_F64, p->collision == LBM_MRT);
+        if (const char* e = std::getenv("LBM_MULTI")) {   // steps per launch, 1 for one each
             const int v = std::atoi(e);
-            if (v >= 1 && v <= 15) c->multi = v;
+            if (v >= 1 && v <= 15) c->plan = StepPlan{v, 2};
         }
     }
     k.sr = 1;

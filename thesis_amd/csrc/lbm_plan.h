@@ -10,6 +10,45 @@ namespace lbm {
 inline long squares_of(int nx, int ny, int side) { return (long)((nx + side - 1) / side) * ((ny + side - 1) / side); }
 inline long rounds_of(long n, long width) { return (n + width - 1) / width; }
 
+// Steps of a launch: at most `most` (1: one launch a step throughout), and at least
+// `least`; what a call leaves over below that goes one launch a step.
+struct StepPlan {
+    int most, least;
+};
+// The plan with the least time a step among launches of up to `top` steps, where
+// launch(t) < `win` t single; single: one launch for one step.
+template <class Launch> inline StepPlan step_plan(int top, double single, double win, Launch launch) {
+    StepPlan p{1, 2};
+    double best = win * single;
+    for (int t = 2; t <= top; ++t)
+        if (launch(t) / t < best) { best = launch(t) / t; p.most = t; }
+    while (p.least < p.most && launch(p.least) >= win * single * p.least) ++p.least;
+    return p;
+}
+
+// D2Q9 lattice of nx x ny nodes, nf of them not solid, FP64 or FP32 (lbm_multi2.hip).
+//
+// One step takes 5.2 us and 24 ns a thousand fluid nodes in FP64, 15.5 in FP32 (256 x
+// 64 5.5 us, 1400 x 700 29.6 / 20.8, 2048 x 2048 105 / 68, 0.4 of them fluid 46 / 30).
+// A launch of t steps works on the whole box, solid or not: squares of 32 - 2t inner
+// nodes a side.  Up to 256 of them have a CU each and cost 7 + 1.65 t us (FP32 5.6 +
+// 1.1 t), more go in rounds of 256 of 6 + 1.25 t us (FP32 2.6 + 0.65 t and 4 for the
+// launch); with MRT a quarter more.  Measured a step at t = 1, 2, 3, 4, 5, 6, 8, 12:
+// FP64 256 x 64 5.5, 6.0, 4.0, 3.5, 3.2, 3.0, 2.5, 2.1 (12 chosen), 500 x 120 6.2, 5.0,
+// 4.2, 3.6, 3.3, 3.0, 2.7, 6.0 (8), 1021 x 256 10.8, 9.5, 7.5, 6.3, 7.4, 7.6, 8.6, 22 (4);
+// 2048 x 2048 FP64 105, 99, 82, 72, 75, 78, 106, 313 (4), of which 0.6 fluid 64, 84, 74,
+// 74 (1), FP32 of which 0.4 fluid 30, 39, 35, 36 (1).
+inline StepPlan flow2_plan(int nx, int ny, size_t nf, bool f64, bool mrt) {
+    const double single = 5.2 + (f64 ? 24e-6 : 15.5e-6) * (double)nf;
+    return step_plan(14, single, 1.0, [&](int t) {
+        const long sq = squares_of(nx, ny, 32 - 2 * t), r = rounds_of(sq, 256);
+        const double c = sq <= 256 ? (f64 ? 7.0 + 1.65 * t : 5.6 + 1.1 * t)
+                         : f64     ? (double)r * (6.0 + 1.25 * t)
+                                   : 4.0 + (double)r * (2.6 + 0.65 * t);
+        return mrt ? 1.25 * c : c;
+    });
+}
+
 // Steps a barrier of a batch that checks its residuals every `every` steps, the
 // squares of all instances at that count, and the workgroups of the grid.
 //
