@@ -142,7 +142,7 @@ lbm_status run_steps(lbm_ctx* c, int64_t nsteps, bool macros_last = true, hipEve
     while (c->plan.most > 1 && !ev_after && nsteps - 1 - k >= c->plan.least) {
         const int m = (int)std::min<int64_t>(c->plan.most, nsteps - 1 - k);
         hipError_t e = launch_multi2(c->p.storage, c->p.collision, c->kp, c->P[c->cur], c->P[c->cur ^ 1], c->node,
-                                     c->cidx, fields(c), m, c->plan.most, c->stream);
+                                     c->cidx, fields(c), m, c->stream);
         if (e != hipSuccess) return fail(c, LBM_EDEVICE, "step launch: %s", hipGetErrorString(e));
         c->cur ^= 1;
         k += m;

@@ -101,9 +101,9 @@ hipError_t launch_step(int q, int storage, int collision, bool open, const KPara
 hipError_t launch_edge(int storage, int collision, const KParams& kp, const void* src, void* dst,
                        const uint32_t* cidx, const Fields& fl, bool write_macros, hipStream_t st);
 // D2Q9, FP64 or FP32: `steps` steps in one launch over squares of 32 x 32 nodes
-// with a frame of halo >= steps recomputed nodes (tile layout, node-local faces).
+// with a frame of `steps` recomputed nodes (tile layout, node-local faces).
 hipError_t launch_multi2(int storage, int collision, const KParams& kp, const void* src, void* dst,
-                         const uint32_t* node, const uint32_t* cidx, const Fields& fl, int steps, int halo,
+                         const uint32_t* node, const uint32_t* cidx, const Fields& fl, int steps,
                          hipStream_t st);
 hipError_t launch_recon(int q, int storage, bool open, const KParams& kp, const void* src,
                         const uint32_t* node, const uint32_t* cidx, Fields fl, hipStream_t st);

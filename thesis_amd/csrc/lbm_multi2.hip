@@ -5,7 +5,7 @@
 // arithmetic.  Here a workgroup takes a square of 32 x 32 nodes, one a thread,
 // pulls the post-collision populations of the square once, advances them `steps`
 // steps with the streamed populations in LDS and writes the inner nodes: after
-// step s the nodes s from the rim are still exact, so a frame of `halo` >= steps
+// step s the nodes s from the rim are still exact, so a frame of `steps`
 // nodes is recomputed by the neighbouring squares instead of being exchanged.
 // The node update is the step's own (walls, Zou-He faces, moments, collision), so
 // the bits are too.
@@ -27,14 +27,14 @@ __global__ __launch_bounds__(kSquare, S == 1 && FULL ? 8 : 4) void k_multi2(cons
                                                    typename Io<D2Q9, S>::raw* __restrict__ dst,
                                                    const uint32_t* __restrict__ node,
                                                    const uint32_t* __restrict__ cidx, KParams kp, Fields fl, int steps,
-                                                   int halo, uint32_t tx) {
+                                                   uint32_t tx) {
     using L = D2Q9;
     using T = typename Io<L, S>::T;
     __shared__ T lds[8][kSquare];
     const int tid = threadIdx.x, lx = tid & (kSide - 1), ly = tid / kSide;
-    const int in = kSide - 2 * halo, nx = kp.nx, ny = kp.ny;
+    const int in = kSide - 2 * steps, nx = kp.nx, ny = kp.ny;
     const uint32_t b = xcd_block(blockIdx.x, gridDim.x, kp.xcd_shift, kp.xchunk_shift), by = b / tx;
-    const int ux = (int)(b - by * tx) * in - halo + lx, uy = (int)by * in - halo + ly;
+    const int ux = (int)(b - by * tx) * in - steps + lx, uy = (int)by * in - steps + ly;
     // periodic axes wrap (boxes smaller than the frame too)
     int x = ux, y = uy;
     if (kp.per[0]) { x %= nx; x = x < 0 ? x + nx : x; }
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(kSquare, S == 1 && FULL ? 8 : 4) void k_multi2(cons
     fn.vbc = ub + 1;
     square_steps<T, C>(kp, fn, idx, live, nd, ln.x, ln.y, steps, lds, p);
     const int rim = min(min(lx, kSide - 1 - lx), min(ly, kSide - 1 - ly));
-    if (live && rim >= halo && ux < nx && uy < ny) {   // ux, uy >= 0 inside the frame
+    if (live && rim >= steps && ux < nx && uy < ny) {   // ux, uy >= 0 inside the frame
 #pragma unroll
         for (int i = 0; i < L::Q; ++i) sto(dst, tslot<L>(i, own), Io<L, S>::pk(p[i], i));
     }
@@ -66,13 +66,13 @@ __global__ __launch_bounds__(kSquare, S == 1 && FULL ? 8 : 4) void k_multi2(cons
 
 template <int S, int C>
 static hipError_t multi_t(const KParams& kp, const void* src, void* dst, const uint32_t* node, const uint32_t* cidx,
-                          const Fields& fl, int steps, int halo, hipStream_t st) {
+                          const Fields& fl, int steps, hipStream_t st) {
     using raw = typename Io<D2Q9, S>::raw;
-    const int in = kSide - 2 * halo;
+    const int in = kSide - 2 * steps;
     const uint32_t tx = (uint32_t)(kp.nx + in - 1) / in, ty = (uint32_t)(kp.ny + in - 1) / in;
     auto go = [&](auto k) {
         hipLaunchKernelGGL(k, dim3(tx * ty), dim3(kSquare), 0, st, (const raw*)src, (raw*)dst, node, cidx, kp, fl, steps,
-                           halo, tx);
+                           tx);
     };
     if (S == 1 && tx * ty > 256) go(k_multi2<S, C, true>);
     else go(k_multi2<S, C, false>);
@@ -80,20 +80,19 @@ static hipError_t multi_t(const KParams& kp, const void* src, void* dst, const u
 }
 
 hipError_t launch_multi2(int storage, int collision, const KParams& kp, const void* src, void* dst,
-                         const uint32_t* node, const uint32_t* cidx, const Fields& fl, int steps, int halo,
-                         hipStream_t st) {
-    if (steps < 1 || steps > halo || 2 * halo >= kSide || storage > 1) return hipErrorInvalidValue;
+                         const uint32_t* node, const uint32_t* cidx, const Fields& fl, int steps, hipStream_t st) {
+    if (steps < 1 || 2 * steps >= kSide || storage > 1) return hipErrorInvalidValue;
     if (storage == 0) {
         switch (collision) {
-        case 0: return multi_t<0, 0>(kp, src, dst, node, cidx, fl, steps, halo, st);
-        case 1: return multi_t<0, 1>(kp, src, dst, node, cidx, fl, steps, halo, st);
-        default: return multi_t<0, 2>(kp, src, dst, node, cidx, fl, steps, halo, st);
+        case 0: return multi_t<0, 0>(kp, src, dst, node, cidx, fl, steps, st);
+        case 1: return multi_t<0, 1>(kp, src, dst, node, cidx, fl, steps, st);
+        default: return multi_t<0, 2>(kp, src, dst, node, cidx, fl, steps, st);
         }
     }
     switch (collision) {
-    case 0: return multi_t<1, 0>(kp, src, dst, node, cidx, fl, steps, halo, st);
-    case 1: return multi_t<1, 1>(kp, src, dst, node, cidx, fl, steps, halo, st);
-    default: return multi_t<1, 2>(kp, src, dst, node, cidx, fl, steps, halo, st);
+    case 0: return multi_t<1, 0>(kp, src, dst, node, cidx, fl, steps, st);
+    case 1: return multi_t<1, 1>(kp, src, dst, node, cidx, fl, steps, st);
+    default: return multi_t<1, 2>(kp, src, dst, node, cidx, fl, steps, st);
     }
 }
 
