@@ -28,6 +28,11 @@ int main() {
             if (std::scanf("%d %d %zu %d %d", &nx, &ny, &nf, &f64, &mrt) != 5) return 1;
             const lbm::StepPlan p = lbm::flow2_plan(nx, ny, nf, f64 != 0, mrt != 0);
             std::printf("%d %d\n", p.most, p.least);
+        } else if (!std::strcmp(what, "cg2")) {
+            int nx, ny, ho, enh, f64;
+            if (std::scanf("%d %d %d %d %d", &nx, &ny, &ho, &enh, &f64) != 5) return 1;
+            const lbm::StepPlan p = lbm::cg2_plan(nx, ny, ho != 0, enh != 0, f64 != 0);
+            std::printf("%d %d\n", p.most, p.least);
         } else {
             return 1;
         }

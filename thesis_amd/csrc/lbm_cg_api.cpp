@@ -2,6 +2,7 @@
 #include "lbm.h"
 #include "lbm_cg.h"
 #include "lbm_hostcopy.h"
+#include "lbm_plan.h"
 
 #include <hip/hip_runtime.h>
 
@@ -37,7 +38,7 @@ struct lbm_cg_ctx {
     void* psi = nullptr;         // 3 N phase field, density, red density (D3Q19)
     double* fout = nullptr;      // 2 q N: populations in and out
     double* partials = nullptr;
-    int multi = 1;               // D2Q9, periodic, FP64 or FP32: most steps of one launch
+    lbm::StepPlan plan{1, 2};    // D2Q9, periodic, FP64 or FP32: steps of one launch
     bool walls = false;          // walls or body force: the reference-order path (lbm_cgw.hip)
     bool fused_walls = false;    // of these D2Q9 FP64: one launch a step, from P[cur] and mac to P[cur ^ 1] and mac2
     lbm::cg::WallParams wp{};
@@ -84,29 +85,6 @@ int cg3_zchunk(int nx, int ny, int nz, int rows, int storage) {
     for (int zc = most; zc >= 1; --zc) {
         const long rounds = (tiles * ((nz + zc - 1) / zc) + cus - 1) / cus, c = rounds * (zc + 2);
         if (cost < 0 || c < cost) { cost = c; best = zc; }
-    }
-    return best;
-}
-// Steps per launch of a periodic D2Q9 box (k_cg_multi): t steps advance 32 - 2 halo
-// nodes a side, halo = t (1 + H) - 1, and cost, where every square has a CU of its own
-// (up to 256), 6 + 2.6 t us (FP32 5 + 2 t); beyond, each round of 256 squares
-// 13.5 + 1.3 t us, in FP32 each round of 512 (two a CU) 11 + 1.6 t us.  The t with the
-// least a step.  Measured per step at t = 1, 2, 3, 4, 5, 6, 8-point stencil: FP64
-// 250 x 187 8.1, 6.2, 5.5, 4.9, 4.5, 7.3 (5 chosen), 512 x 512 17.6, 15.2, 16.1, 17.7,
-// 22.9, 37.5 (2), 1024 x 700 50.5, 41.1, 36.5, 40.8, 58.8, 99.9 (3); FP32 512 x 512
-// 10.3, 8.4, 8.7, 9.8, 12.4, 19.6 (2), 1024 x 700 30.7, 21.3, 17.7, 21.3, 29.6, 50.6 (3);
-// 24-point FP64 512 x 512 19.4, 19.6, 18.8, 41.9, 194 (3), 1024 x 700 54.5, 44.6, 51.5 (2).
-int cg_multi_steps(int nx, int ny, bool ho, bool f64) {
-    int best = 1;
-    double cost = 0;
-    for (int t = 2; t <= (ho ? 5 : 8); ++t) {
-        const int in = 32 - 2 * (t * (ho ? 3 : 2) - 1);
-        const double squares = (double)((nx + in - 1) / in) * ((ny + in - 1) / in);
-        const double one = f64 ? 6.0 + 2.6 * t : 5.0 + 2.0 * t;
-        const double c = (squares <= 256.0 ? one
-                          : f64            ? std::ceil(squares / 256.0) * (13.5 + 1.3 * t)
-                                           : std::ceil(squares / 512.0) * (11.0 + 1.6 * t)) / t;
-        if (best == 1 || c < cost) { cost = c; best = t; }
     }
     return best;
 }
@@ -174,10 +152,10 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
     c->walls = walls;
     c->fused_walls = walls && !three_d && p->storage == LBM_STORE_F64;
     if (!walls && !three_d && p->storage != LBM_STORE_F16) {   // LBM_CG_MULTI: steps per launch, 1 for one each
-        c->multi = cg_multi_steps(p->nx, p->ny, p->high_order != 0, p->storage == LBM_STORE_F64);
+        c->plan = lbm::cg2_plan(p->nx, p->ny, p->high_order != 0, p->enhanced != 0, p->storage == LBM_STORE_F64);
         if (const char* e = std::getenv("LBM_CG_MULTI")) {
             const int v = std::atoi(e);
-            if (v >= 1 && v <= (p->high_order ? 5 : 8)) c->multi = v;
+            if (v >= 1 && v <= (p->high_order ? 5 : 8)) c->plan = lbm::StepPlan{v, 2};
         }
     }
     c->wp.cp = k;
@@ -272,10 +250,10 @@ lbm_status lbm_cg_init_f(lbm_cg_ctx* c, const double* r_f, const double* b_f) {
 // and get_f reads the state before it from the other buffer.
 static lbm_status cg_run(lbm_cg_ctx* c, int64_t nsteps) {
     int64_t k = 0;
-    while (c->multi > 1 && nsteps - 1 - k > 1) {
-        const int m = (int)std::min<int64_t>(c->multi, nsteps - 1 - k);
-        CGCHK(c, lbm::cg_launch_multi(c->p.storage, c->p.high_order, c->P[c->cur], c->P[c->cur ^ 1], c->cp, m, c->multi,
-                                      c->stream));
+    while (c->plan.most > 1 && nsteps - 1 - k >= c->plan.least) {
+        const int m = (int)std::min<int64_t>(c->plan.most, nsteps - 1 - k);
+        CGCHK(c, lbm::cg_launch_multi(c->p.storage, c->p.high_order, c->P[c->cur], c->P[c->cur ^ 1], c->cp, m,
+                                      c->plan.most, c->stream));
         c->cur ^= 1;
         k += m;
     }

@@ -3,6 +3,7 @@
 // tests/test_plan.py holds them against measured times on any machine.
 #pragma once
 #include <algorithm>
+#include <cmath>
 #include <cstddef>
 
 namespace lbm {
@@ -46,6 +47,39 @@ inline StepPlan flow2_plan(int nx, int ny, size_t nf, bool f64, bool mrt) {
                          : f64     ? (double)r * (6.0 + 1.25 * t)
                                    : 4.0 + (double)r * (2.6 + 0.65 * t);
         return mrt ? 1.25 * c : c;
+    });
+}
+
+// Periodic two-phase D2Q9 box, FP64 or FP32, ho: 24-point stencil, enh: enhanced model
+// (lbm_cg.hip).
+//
+// One step is a launch of tiles of 32 x 16 nodes: up to 256 of them 8.2 us (FP32 6.6),
+// more in rounds of 512 of 18 us (10.5), where there are many 7.4 us (4.45) for each
+// 256; a twentieth more with the 24-point stencil.  A launch of t steps is one of squares
+// of 32 - 2 halo inner nodes, halo = t (1 + H) - 1, and costs, where every square has a
+// CU of its own (up to 256), 6 + 2.6 t us (FP32 5 + 2 t); beyond, each round of 256
+// squares 14.5 + 0.9 t us, with the 24-point stencil 12.6 + 0.7 t, in FP32 each round of
+// 512 (two a CU) 12.4 + t us and the launch 4, with the 24-point stencil 12 + 0.9 t and 2; the enhanced model adds 6 %, 12 % with the 24-point
+// stencil.  Measured per step at t = 1, 2, 3, 4, 5, 6, 8-point stencil: FP64 250 x 187
+// 8.1, 6.2, 5.5, 4.9, 4.5, 7.3 (5 chosen), 512 x 512 17.6, 15.2, 16.1, 17.7, 22.9, 37.5
+// (2), 1024 x 700 50.5, 41.1, 36.5, 40.8, 58.8, 99.9 (3); FP32 512 x 512 10.3, 8.4, 8.7,
+// 9.8, 12.4, 19.6 (2), 1024 x 700 30.7, 21.3, 17.7, 21.3, 29.6, 50.6 (3); 24-point FP64
+// 512 x 512 19.2, 20.0, 19.5, 41.7 (1), with the enhanced model 19.0, 21.9, 22.0 (1),
+// 1024 x 1024 76, 66, 75 (2), 2048 x 2048 enhanced 258, 278, 329 (1); 8-point 2048 x 2048
+// 245, 232, 205, 223 (3).
+inline StepPlan cg2_plan(int nx, int ny, bool ho, bool enh, bool f64) {
+    const double x = (double)((nx + 31) / 32) * ((ny + 15) / 16) / 256.0;
+    double single = f64 ? 8.2 : 6.6;
+    if (x > 1.0) single = f64 ? std::min(18.0 * std::ceil(x / 2), 10.0 + 7.4 * x) : std::min(10.5 * std::ceil(x / 2), 6.0 + 4.45 * x);
+    if (ho) single *= f64 ? 1.05 : 1.08;
+    return step_plan(ho ? 5 : 8, single, 1.0, [&](int t) {
+        const long sq = squares_of(nx, ny, 32 - 2 * (t * (ho ? 3 : 2) - 1));
+        const double c = sq <= 256 ? (f64 ? 6.0 + 2.6 * t : 5.0 + 2.0 * t)
+                         : !f64    ? (ho ? 2.0 + (double)rounds_of(sq, 512) * (12.0 + 0.9 * t)
+                                         : 4.0 + (double)rounds_of(sq, 512) * (12.4 + 1.0 * t))
+                         : ho      ? (double)rounds_of(sq, 256) * (12.6 + 0.7 * t)
+                                   : (double)rounds_of(sq, 256) * (14.5 + 0.9 * t);
+        return enh ? (ho && f64 ? 1.12 : 1.06) * c : c;
     });
 }
 
