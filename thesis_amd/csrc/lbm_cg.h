@@ -90,8 +90,8 @@ __device__ inline T cdot(int kx, int ky, int kz, T a, T b, T c) {
 // D2Q9 (lbm_cg.hip)
 hipError_t cg_launch_step(int storage, int ho, const void* src, void* dst, const cg::CgParams& cp, double* mac,
                           bool wm, hipStream_t st);
-// `steps` <= most steps in one launch (FP64, FP32), without macros; the frame is sized for `most`
-hipError_t cg_launch_multi(int storage, int ho, const void* src, void* dst, const cg::CgParams& cp, int steps, int most,
+// `steps` steps in one launch (FP64, FP32), without macros
+hipError_t cg_launch_multi(int storage, int ho, const void* src, void* dst, const cg::CgParams& cp, int steps,
                            hipStream_t st);
 hipError_t cg_launch_init(int storage, int ho, void* dst, const cg::CgParams& cp, const double* rr,
                           const double* rb, const double* rf, const double* bf, double* mac, hipStream_t st);

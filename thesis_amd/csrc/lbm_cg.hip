@@ -236,7 +236,7 @@ __global__ __launch_bounds__(THREADS) void k_cg_step(const typename CIo<S>::raw*
 // 32 x 32 nodes, one a thread, pulls their populations once, advances them `steps`
 // steps with the moving links changing hands in LDS and stores the inner nodes.  The
 // pull makes every node's streamed state exact; a collision then costs H rings (the
-// gradient) and each further streaming one more, so a frame of `halo` >=
+// gradient) and each further streaming one more, so a frame of `halo` =
 // steps (1 + H) - 1 nodes is recomputed by the neighbouring squares.  The node update
 // is k_cg_step's on the same values: the results are its bits.  FP16 storage stays
 // with k_cg_step: there the conversion of a pulled value is fused into the density's
@@ -453,10 +453,10 @@ hipError_t cg_launch_step(int storage, int ho, const void* src, void* dst, const
     return hipGetLastError();
 }
 
-hipError_t cg_launch_multi(int storage, int ho, const void* src, void* dst, const cg::CgParams& cp, int steps, int most,
+hipError_t cg_launch_multi(int storage, int ho, const void* src, void* dst, const cg::CgParams& cp, int steps,
                            hipStream_t st) {
-    const int halo = most * (ho ? 3 : 2) - 1, in = cg::SIDE - 2 * halo;
-    if (steps < 1 || steps > most || in < 1 || storage < 0 || storage > 1) return hipErrorInvalidValue;
+    const int halo = steps * (ho ? 3 : 2) - 1, in = cg::SIDE - 2 * halo;
+    if (steps < 1 || in < 1 || storage < 0 || storage > 1) return hipErrorInvalidValue;
     const uint32_t tx = (uint32_t)(cp.nx + in - 1) / in, ty = (uint32_t)(cp.ny + in - 1) / in;
 #define CG_M(S_, H_, E_, F_)                                                                                 \
     hipLaunchKernelGGL((cg::k_cg_multi<S_, H_, E_, F_>), dim3(tx * ty), dim3(cg::SQ), 0, st,                 \

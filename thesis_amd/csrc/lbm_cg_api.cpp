@@ -253,7 +253,7 @@ static lbm_status cg_run(lbm_cg_ctx* c, int64_t nsteps) {
     while (c->plan.most > 1 && nsteps - 1 - k >= c->plan.least) {
         const int m = (int)std::min<int64_t>(c->plan.most, nsteps - 1 - k);
         CGCHK(c, lbm::cg_launch_multi(c->p.storage, c->p.high_order, c->P[c->cur], c->P[c->cur ^ 1], c->cp, m,
-                                      c->plan.most, c->stream));
+                                      c->stream));
         c->cur ^= 1;
         k += m;
     }
