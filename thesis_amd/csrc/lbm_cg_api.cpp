@@ -35,7 +35,7 @@ struct lbm_cg_ctx {
     double* mac = nullptr;       // 6 N: rho_r, rho_b, rho, u, v, w
     double* mac2 = nullptr;      // the macros of the step before (fused_walls)
     double* rr0 = nullptr;       // 2 N initial densities
-    void* psi = nullptr;         // 3 N phase field, density, red density (D3Q19)
+    void* psi = nullptr;         // D3Q19: phase field, density and red density, N each (the last where it is read)
     double* fout = nullptr;      // 2 q N: populations in and out
     double* partials = nullptr;
     lbm::StepPlan plan{1, 2};    // D2Q9, periodic, FP64 or FP32: steps of one launch
@@ -167,10 +167,13 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreate(&c->ev0) == hipSuccess && hipEventCreate(&c->ev1) == hipSuccess;
     const size_t pb = 2 * (size_t)q * plane * sbytes(p->storage);
+    // in the step's type: phase field and density, and the red density of the FP64 and FP32 two-launch step
+    const bool red = !walls && k.zchunk == 0 && p->storage != LBM_STORE_F16;
+    const size_t psi = (red ? 3 : 2) * n * (p->storage == LBM_STORE_F64 ? 8 : 4);
     ok = ok && hipMalloc(&c->P[0], pb) == hipSuccess && hipMalloc(&c->P[1], pb) == hipSuccess &&
          hipMalloc((void**)&c->mac, 6 * n * 8) == hipSuccess && hipMalloc((void**)&c->rr0, 2 * n * 8) == hipSuccess &&
          hipMalloc((void**)&c->partials, (size_t)kRedBlocks * lbm::cg::NRED * 8) == hipSuccess &&
-         (!three_d || hipMalloc(&c->psi, 3 * n * 8) == hipSuccess) &&
+         (!three_d || hipMalloc(&c->psi, psi) == hipSuccess) &&
          hipMemset(c->mac + 5 * n, 0, n * 8) == hipSuccess &&
          (!c->fused_walls || (hipMalloc((void**)&c->mac2, 6 * n * 8) == hipSuccess &&
                               hipMemset(c->mac2 + 5 * n, 0, n * 8) == hipSuccess));
