@@ -267,7 +267,7 @@ __device__ inline bool node_of(const CgParams& cp, int& x, int& y, int& z) {
 // pulls the deviations alone (FP32 per step, both launches: 128^3 104-point 198 to
 // 179 us, 256^3 1483 to 1346, 192 x 96 x 61 18-point 90 to 77, 64 x 96 x 160 76 to 67).
 // Not so in FP16, whose step sums the rounded products of its conversion.  Bound by
-// memory: 4 of 6 values a link move now.
+// memory: 5 of 6 values a link move now.
 template <int S, bool E>
 __global__ __launch_bounds__(BX * BY) void k_cg3_psi(const typename CIo<S>::raw* __restrict__ src, CgParams cp,
                                                      typename CIo<S>::T* __restrict__ psi) {

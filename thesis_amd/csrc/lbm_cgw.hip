@@ -278,7 +278,7 @@ __device__ inline double quot(double a, double b, double ib) {
 //
 // What bounds a box that fits the caches is one wavefront's chain of FP64
 // instructions (250 x 187: 47 k nodes, a wavefront a SIMD): the two launches
-// took 15.7 us a step there, this one 7.9 us.  Larger ones move 48 instead of 92
+// took 15.7 us a step there, this one 7.9 us.  Larger ones move 46 instead of 85
 // values a node: 1024 x 700 91 to 56 us.
 template <int BX, int BY, int H, bool E>
 __global__ __launch_bounds__(BX * BY) void k_cgw_step64(const double* __restrict__ P, double* __restrict__ Pn,
@@ -704,7 +704,7 @@ hipError_t cgw_launch_step(int storage, const void* P, void* Pc, double* mac, co
 #undef CGW3_
         return hipGetLastError();
     }
-    // D2Q9 here: FP32 (FP64 goes by cgw_launch_step64)
+    if (storage != 1) return hipErrorInvalidValue;   // D2Q9 here: FP32 (FP64 goes by cgw_launch_step64)
     if (wp.cp.enhanced)
         hipLaunchKernelGGL((cgw::k_cgw_collide<float, true>), dim3(blocks), dim3(256), 0, st, (const float*)P,
                            (float*)Pc, mac, wp);
