@@ -885,8 +885,8 @@ __device__ inline void outlet3_local(const KParams& kp, const Fields& fl, size_t
 }
 template <class L, int S, bool OPEN>
 __device__ inline void outlet3d(const typename Io<L, S>::raw* __restrict__ src, const KParams& kp, const Fields& fl,
-                                const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ nodew, bool compact,
-                                int x, int y, int z, size_t idx, uint32_t cls, typename Io<L, S>::T* h) {
+                                const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ node, int x, int y,
+                                int z, size_t idx, uint32_t cls, typename Io<L, S>::T* h) {
     using T = typename Io<L, S>::T;
     if (L::Q != 19 || !is_outlet3(cls)) return;
     T f[L::Q];   // a local copy keeps the caller's populations in registers across the switch
@@ -910,10 +910,9 @@ __device__ inline void outlet3d(const typename Io<L, S>::raw* __restrict__ src, 
         if (a == kNone || b == kNone) return;
         const int dx = A == 0 ? G : 0, dy = A == 1 ? G : 0, dz = A == 2 ? G : 0;
         T ha[L::Q], hb[L::Q];
-        inflow_state<L, S, OPEN>(src, kp, fl, cidx, a, compact ? nodew[a] : nodew[i1], x + dx, y + dy, z + dz, i1, ha);
+        inflow_state<L, S, OPEN>(src, kp, fl, cidx, a, node[i1], x + dx, y + dy, z + dz, i1, ha);
         if (second)
-            inflow_state<L, S, OPEN>(src, kp, fl, cidx, b, compact ? nodew[b] : nodew[i2], x + 2 * dx, y + 2 * dy,
-                                     z + 2 * dz, i2, hb);
+            inflow_state<L, S, OPEN>(src, kp, fl, cidx, b, node[i2], x + 2 * dx, y + 2 * dy, z + 2 * dz, i2, hb);
         switch (cls) {
         case PRES_E: extrap_mix<L, T, 0, -1>(f, ha, hb, second); break;
         case OUT_W: extrap_mix<L, T, 0, 1>(f, ha, hb, second); break;

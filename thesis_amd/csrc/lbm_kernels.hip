@@ -482,7 +482,7 @@ __device__ inline void post_boundary(const typename Io<L, S>::raw* __restrict__ 
         outlet_extrap<L, S, OPEN>(src, kp, fl, cidx, node, false, x, y, z, idx, h);
     }
     if (OPEN && L::Q == 19) {
-        if (is_outlet3(cls)) outlet3d<L, S, OPEN>(src, kp, fl, cidx, node, false, x, y, z, idx, cls, h);
+        if (is_outlet3(cls)) outlet3d<L, S, OPEN>(src, kp, fl, cidx, node, x, y, z, idx, cls, h);
         sym3d<L, T>(cls, h);
     }
 }
