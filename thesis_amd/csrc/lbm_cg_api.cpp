@@ -32,6 +32,7 @@ struct lbm_cg_ctx {
     int cur = 0;
     int dev = 0;                 // device current at creation
     int64_t steps = -1;
+    double* macs = nullptr;      // the allocation of mac and mac2
     double* mac = nullptr;       // 6 N: rho_r, rho_b, rho, u, v, w
     double* mac2 = nullptr;      // the macros of the step before (fused_walls)
     double* rr0 = nullptr;       // 2 N initial densities
@@ -167,20 +168,21 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreate(&c->ev0) == hipSuccess && hipEventCreate(&c->ev1) == hipSuccess;
     const size_t pb = 2 * (size_t)q * plane * sbytes(p->storage);
+    const size_t sets = c->fused_walls ? 2 : 1;   // one allocation and one clearing: a second of each took 40 us
     // in the step's type: phase field and density, and the red density of the FP64 and FP32 two-launch step
     const bool red = !walls && k.zchunk == 0 && p->storage != LBM_STORE_F16;
     const size_t psi = (red ? 3 : 2) * n * (p->storage == LBM_STORE_F64 ? 8 : 4);
     ok = ok && hipMalloc(&c->P[0], pb) == hipSuccess && hipMalloc(&c->P[1], pb) == hipSuccess &&
-         hipMalloc((void**)&c->mac, 6 * n * 8) == hipSuccess && hipMalloc((void**)&c->rr0, 2 * n * 8) == hipSuccess &&
+         hipMalloc((void**)&c->macs, sets * 6 * n * 8) == hipSuccess && hipMalloc((void**)&c->rr0, 2 * n * 8) == hipSuccess &&
          hipMalloc((void**)&c->partials, (size_t)kRedBlocks * lbm::cg::NRED * 8) == hipSuccess &&
          (!three_d || hipMalloc(&c->psi, psi) == hipSuccess) &&
-         hipMemset(c->mac + 5 * n, 0, n * 8) == hipSuccess &&
-         (!c->fused_walls || (hipMalloc((void**)&c->mac2, 6 * n * 8) == hipSuccess &&
-                              hipMemset(c->mac2 + 5 * n, 0, n * 8) == hipSuccess));
+         hipMemset(c->macs + 5 * n, 0, (sets * 6 - 5) * n * 8) == hipSuccess;   // w, which no 2D step writes
     if (!ok) {
         lbm_cg_destroy(c);
         return LBM_ENOMEM;
     }
+    c->mac = c->macs;
+    if (c->fused_walls) c->mac2 = c->macs + 6 * n;
     *out = c;
     return LBM_OK;
 }
@@ -188,7 +190,7 @@ lbm_status lbm_cg_create(const lbm_cg_params* p, lbm_cg_ctx** out) {
 void lbm_cg_destroy(lbm_cg_ctx* c) {
     if (!c) return;
     if (c->stream) hipStreamSynchronize(c->stream);
-    void* b[] = {c->P[0], c->P[1], c->mac, c->mac2, c->rr0, c->psi, c->fout, c->partials};
+    void* b[] = {c->P[0], c->P[1], c->macs, c->rr0, c->psi, c->fout, c->partials};
     for (void* x : b)
         if (x) hipFree(x);
     if (c->ev0) hipEventDestroy(c->ev0);
