@@ -324,7 +324,8 @@ lbm_status lbm_batch_run(lbm_batch* b, double tol, int32_t check_every, int64_t 
     BCHK(b, hipMemcpyAsync(b->bs.res, rinf.data(), sizeof(double) * n, h2d, b->stream));
     BCHK(b, hipMemcpyAsync(b->bs.remaining, &remaining, sizeof(int), h2d, b->stream));
     // the last step is a check too
-    const BatchPlan plan = batch_plan(b->hinst.data(), n, b->ntiles, b->blocks, std::min<int64_t>(check_every, max_steps));
+    const BatchPlan plan =
+        batch_plan(b->hinst.data(), n, b->ntiles, b->blocks, (long)std::min<int64_t>(check_every, max_steps));
     if (plan.halo > 1 && plan.halo != b->halo) {
         uint32_t at = 0;
         const int side = 32 - 2 * plan.halo;

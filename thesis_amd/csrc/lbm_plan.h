@@ -59,18 +59,20 @@ inline StepPlan flow2_plan(int nx, int ny, size_t nf, bool f64, bool mrt) {
 // of 32 - 2 halo inner nodes, halo = t (1 + H) - 1, and costs, where every square has a
 // CU of its own (up to 256), 6 + 2.6 t us (FP32 5 + 2 t); beyond, each round of 256
 // squares 14.5 + 0.9 t us, with the 24-point stencil 12.6 + 0.7 t, in FP32 each round of
-// 512 (two a CU) 12.4 + t us and the launch 4, with the 24-point stencil 12 + 0.9 t and 2; the enhanced model adds 6 %, 12 % with the 24-point
-// stencil.  Measured per step at t = 1, 2, 3, 4, 5, 6, 8-point stencil: FP64 250 x 187
-// 8.1, 6.2, 5.5, 4.9, 4.5, 7.3 (5 chosen), 512 x 512 17.6, 15.2, 16.1, 17.7, 22.9, 37.5
-// (2), 1024 x 700 50.5, 41.1, 36.5, 40.8, 58.8, 99.9 (3); FP32 512 x 512 10.3, 8.4, 8.7,
-// 9.8, 12.4, 19.6 (2), 1024 x 700 30.7, 21.3, 17.7, 21.3, 29.6, 50.6 (3); 24-point FP64
-// 512 x 512 19.2, 20.0, 19.5, 41.7 (1), with the enhanced model 19.0, 21.9, 22.0 (1),
-// 1024 x 1024 76, 66, 75 (2), 2048 x 2048 enhanced 258, 278, 329 (1); 8-point 2048 x 2048
-// 245, 232, 205, 223 (3).
+// 512 (two a CU) 12.4 + t us and the launch 4, with the 24-point stencil 12 + 0.9 t and
+// 2; the enhanced model adds 6 %, FP64 with the 24-point stencil 12 %.  Measured per step
+// at t = 1, 2, 3, 4, 5, 6, 8-point stencil: FP64 250 x 187 8.2, 6.7, 5.8, 5.1, 4.8, 7.5
+// (5 chosen), 512 x 512 17.8, 15.6, 16.6, 18.1, 23.0, 37.4 (2), 1024 x 1024 69, 58, 54,
+// 59, 84, 140 (3), 2048 x 2048 245, 232, 205, 223, 317, 540 (3); FP32 512 x 512 10.4, 8.9,
+// 9.1, 10.2, 12.8, 19.7 (2), 1024 x 1024 43, 31, 26, 31, 45, 71 (3); 24-point FP64 512 x
+// 512 19.2, 20.0, 19.5, 41.7 (1), with the enhanced model 19.0, 21.9, 22.0 (1), 1024 x
+// 1024 76, 66, 75 (2), 2048 x 2048 enhanced 258, 278, 329 (1).
 inline StepPlan cg2_plan(int nx, int ny, bool ho, bool enh, bool f64) {
     const double x = (double)((nx + 31) / 32) * ((ny + 15) / 16) / 256.0;
     double single = f64 ? 8.2 : 6.6;
-    if (x > 1.0) single = f64 ? std::min(18.0 * std::ceil(x / 2), 10.0 + 7.4 * x) : std::min(10.5 * std::ceil(x / 2), 6.0 + 4.45 * x);
+    if (x > 1.0)
+        single = f64 ? std::min(18.0 * std::ceil(x / 2), 10.0 + 7.4 * x)
+                     : std::min(10.5 * std::ceil(x / 2), 6.0 + 4.45 * x);
     if (ho) single *= f64 ? 1.05 : 1.08;
     return step_plan(ho ? 5 : 8, single, 1.0, [&](int t) {
         const long sq = squares_of(nx, ny, 32 - 2 * (t * (ho ? 3 : 2) - 1));
@@ -114,7 +116,8 @@ inline BatchPlan batch_plan(const Inst* inst, int n, long tiles, int most_blocks
             return s < 2 ? (double)s * single : bar + (double)rounds_of(sq, g) * (6.0 + 1.25 * (double)s);
         };
         const long rest = every - 1, full = t > 1 ? rest / t : 0;
-        const double c = bar + single + (t > 1 ? (double)full * phase(t) + phase(rest - full * t) : (double)rest * single);
+        const double c =
+            bar + single + (t > 1 ? (double)full * phase(t) + phase(rest - full * t) : (double)rest * single);
         if (t == 1) least = 0.95 * c;
         else if (c <= least) { least = c; best = BatchPlan{t, sq, (int)g}; }
     }
