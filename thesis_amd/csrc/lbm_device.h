@@ -835,12 +835,6 @@ __device__ inline void outlet3_face(const KParams& kp, const Fields& fl, size_t 
         return;
     }
 }
-template <class L, class T, int A, int G>
-__device__ inline void extrap_mix(T* f, const T* ha, const T* hb, bool second) {
-#pragma unroll
-    for (int i = 0; i < L::Q; ++i)
-        if (G * cmp<L>(i, A) > 0) f[i] = second ? (T)2 * ha[i] - hb[i] : ha[i];
-}
 // Term k of an extrapolating outlet node's populations: k = 0 its own (all of
 // them), then the unknowns from the nodes upstream, 2 f(x+n) - f(x+2n) (second)
 // or f(x+n).
@@ -883,49 +877,59 @@ __device__ inline void outlet3_local(const KParams& kp, const Fields& fl, size_t
     }
     if (kp.mref) mref_shift<L, T>(f, 1);
 }
-template <class L, int S, bool OPEN>
-__device__ inline void outlet3d(const typename Io<L, S>::raw* __restrict__ src, const KParams& kp, const Fields& fl,
-                                const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ node, int x, int y,
-                                int z, size_t idx, uint32_t cls, typename Io<L, S>::T* h) {
+
+// Post-boundary populations h of non-solid node idx (compact slot own, word nd) from
+// the post-collision state in src: the pull, walls and open faces.  words holds
+// node words by compact index, with DENSE by dense index.  HH, CURVED, EXT: whether the
+// lattice may have wet-node walls, curved walls and extrapolating 3D outlets
+// (kernels for lattices without them leave the code out).
+template <class L, int S, bool OPEN, bool DENSE, bool HH = true, bool CURVED = true, bool EXT = true>
+__device__ inline void post_boundary(const typename Io<L, S>::raw* __restrict__ src, const KParams& kp,
+                                     const Fields& fl, const uint32_t* __restrict__ words,
+                                     const uint32_t* __restrict__ cidx, uint32_t own, uint32_t nd, int x, int y,
+                                     int z, uint32_t idx, typename Io<L, S>::T* h) {
     using T = typename Io<L, S>::T;
-    if (L::Q != 19 || !is_outlet3(cls)) return;
-    T f[L::Q];   // a local copy keeps the caller's populations in registers across the switch
-#pragma unroll
-    for (int i = 0; i < L::Q; ++i) f[i] = h[i];
-    if (kp.outlet == 2 || kp.outlet == 3) {
-        // Extrapolation: the two upstream nodes along the inward normal are
-        // recomputed once, outside the per-face code.
-        const int A = cls == PRES_E || cls == OUT_W ? 0 : (cls == OUT_S || cls == OUT_N ? 1 : 2);
-        const int G = cls == OUT_W || cls == OUT_S || cls == OUT_B ? 1 : -1;
-        const bool second = kp.outlet == 2;
-        const int dims[3] = {kp.nx, kp.ny, kp.nz};
-        const int pa = A == 0 ? x : A == 1 ? y : z;
-        const int reach = pa + G * (second ? 2 : 1);
-        if (reach < 0 || reach >= dims[A < 1 ? 0 : (A < 2 ? 1 : 2)]) return;
-        const size_t stride = A == 0 ? 1 : A == 1 ? (size_t)kp.nx : (size_t)kp.nx * kp.ny;
-        const size_t i1 = G > 0 ? idx + stride : idx - stride;
-        const size_t i2 = G > 0 ? idx + 2 * stride : idx - 2 * stride;
-        const uint32_t a = cidx[i1];
-        const uint32_t b = second ? cidx[i2] : 0u;
-        if (a == kNone || b == kNone) return;
-        const int dx = A == 0 ? G : 0, dy = A == 1 ? G : 0, dz = A == 2 ? G : 0;
-        T ha[L::Q], hb[L::Q];
-        inflow_state<L, S, OPEN>(src, kp, fl, cidx, a, node[i1], x + dx, y + dy, z + dz, i1, ha);
-        if (second)
-            inflow_state<L, S, OPEN>(src, kp, fl, cidx, b, node[i2], x + 2 * dx, y + 2 * dy, z + 2 * dz, i2, hb);
-        switch (cls) {
-        case PRES_E: extrap_mix<L, T, 0, -1>(f, ha, hb, second); break;
-        case OUT_W: extrap_mix<L, T, 0, 1>(f, ha, hb, second); break;
-        case OUT_S: extrap_mix<L, T, 1, 1>(f, ha, hb, second); break;
-        case OUT_N: extrap_mix<L, T, 1, -1>(f, ha, hb, second); break;
-        case OUT_B: extrap_mix<L, T, 2, 1>(f, ha, hb, second); break;
-        default: extrap_mix<L, T, 2, -1>(f, ha, hb, second); break;
+    const uint32_t cls = nd >> kClsShift;
+    if constexpr (OPEN && L::Q == 19 && EXT) {
+        // An extrapolating outlet node takes its unknowns from the one or two
+        // nodes upstream: the pull, walls and faces of up to three nodes in a
+        // loop, so that their code is there once (three copies become calls,
+        // with the populations in scratch).
+        int nk = 1, dx = 0, dy = 0, dz = 0;
+        if (is_outlet3(cls) && (kp.outlet == 2 || kp.outlet == 3)) {
+            const int A = cls == PRES_E || cls == OUT_W ? 0 : (cls == OUT_S || cls == OUT_N ? 1 : 2);
+            const int G = cls == OUT_W || cls == OUT_S || cls == OUT_B ? 1 : -1;
+            dx = A == 0 ? G : 0; dy = A == 1 ? G : 0; dz = A == 2 ? G : 0;
+            const int n = kp.outlet == 2 ? 2 : 1;
+            const int ex = x + n * dx, ey = y + n * dy, ez = z + n * dz;
+            if (ex >= 0 && ex < kp.nx && ey >= 0 && ey < kp.ny && ez >= 0 && ez < kp.nz) nk = n + 1;
+        }
+        const int step = dx + (dy + dz * kp.ny) * kp.nx;
+        uint32_t oj[3] = {own, 0u, 0u};
+        if (nk > 1) {   // a solid node upstream: the streamed values stay
+            oj[1] = cidx[idx + (uint32_t)step];
+            oj[2] = nk > 2 ? cidx[idx + (uint32_t)(2 * step)] : 0u;
+            if (oj[1] == kNone || oj[2] == kNone) nk = 1;
+        }
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < nk; ++k) {
+            const uint32_t j = k == 0 ? own : k == 1 ? oj[1] : oj[2], ik = idx + (uint32_t)(k * step);
+            T hk[L::Q];
+            inflow_state<L, S, OPEN, HH, CURVED>(src, kp, fl, cidx, j, words[DENSE ? ik : j], x + k * dx, y + k * dy,
+                                                 z + k * dz, ik, hk);
+            extrap_term<L, T>(cls, k, kp.outlet == 2, hk, h);
         }
     } else {
-        outlet3_local<L, S, OPEN>(kp, fl, idx, cls, f);
+        inflow_state<L, S, OPEN, HH, CURVED>(src, kp, fl, cidx, own, nd, x, y, z, idx, h);
     }
-#pragma unroll
-    for (int i = 0; i < L::Q; ++i) h[i] = f[i];
+    if (OPEN && L::Q == 9 && cls == PRES_E) {
+        zou_outlet<L, T>(kp, fl, idx, h);
+        outlet_extrap<L, S, OPEN>(src, kp, fl, cidx, words, !DENSE, x, y, z, idx, h);
+    }
+    if (OPEN && L::Q == 19) {
+        if (is_outlet3(cls) && kp.outlet != 2 && kp.outlet != 3) outlet3_local<L, S, OPEN>(kp, fl, idx, cls, h);
+        sym3d<L, T>(cls, h);
+    }
 }
 
 __device__ inline double recip(double x) { return 1.0 / x; }

@@ -467,26 +467,6 @@ __global__ __launch_bounds__(512) void k_stepr2(const typename Io<L, S>::raw* __
     }
 }
 
-// Post-boundary populations h of non-solid node idx (compact slot own) from
-// the post-collision state in src: the pull, walls and open faces of the step.
-template <class L, int S, bool OPEN>
-__device__ inline void post_boundary(const typename Io<L, S>::raw* __restrict__ src, const KParams& kp,
-                                     const Fields& fl, const uint32_t* __restrict__ node,
-                                     const uint32_t* __restrict__ cidx, uint32_t own, uint32_t nd, int x, int y,
-                                     int z, size_t idx, typename Io<L, S>::T* h) {
-    using T = typename Io<L, S>::T;
-    const uint32_t cls = nd >> kClsShift;
-    inflow_state<L, S, OPEN>(src, kp, fl, cidx, own, nd, x, y, z, idx, h);
-    if (OPEN && L::Q == 9 && cls == PRES_E) {
-        zou_outlet<L, T>(kp, fl, idx, h);
-        outlet_extrap<L, S, OPEN>(src, kp, fl, cidx, node, false, x, y, z, idx, h);
-    }
-    if (OPEN && L::Q == 19) {
-        if (is_outlet3(cls)) outlet3d<L, S, OPEN>(src, kp, fl, cidx, node, x, y, z, idx, cls, h);
-        sym3d<L, T>(cls, h);
-    }
-}
-
 // Post-boundary populations (dense, full, FP64) and moments of the state in src;
 // with fl.fout null only the moments are written.
 template <class L, int S, bool OPEN>
@@ -510,7 +490,7 @@ __global__ __launch_bounds__(256) void k_recon(const typename Io<L, S>::raw* __r
     const uint32_t nd = node[idx];
     const uint32_t cls = nd >> kClsShift;
     T h[L::Q];
-    post_boundary<L, S, OPEN>(src, kp, fl, node, cidx, own, nd, x, y, z, idx, h);
+    post_boundary<L, S, OPEN, true>(src, kp, fl, node, cidx, own, nd, x, y, z, (uint32_t)idx, h);
     T drho, rho, u[3];
     moments<L, T>(kp, cls, h, drho, rho, u);
     if (OPEN) frozen_macros<T>(kp, fl, cls, idx, drho, rho, u);
@@ -691,7 +671,7 @@ __global__ __launch_bounds__(kRedThreads) void k_l2_fused(const typename Io<L, S
         const int x = (int)(i - row * (size_t)kp.nx);
         const int y = (int)(row % (size_t)kp.ny), z = (int)(row / (size_t)kp.ny);
         T h[L::Q];
-        post_boundary<L, S, OPEN>(pc, kp, fl, node, cidx, own, node[i], x, y, z, i, h);
+        post_boundary<L, S, OPEN, true>(pc, kp, fl, node, cidx, own, node[i], x, y, z, (uint32_t)i, h);
 #pragma unroll
         for (int q = 0; q < L::Q; ++q) {
             const T hc = Io<L, S>::ld(pc, paddr<L>(kp, q, own), q);

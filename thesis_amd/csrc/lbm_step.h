@@ -53,8 +53,7 @@ __device__ inline void store_node(typename Io<L, S>::raw* __restrict__ dst, cons
 }
 
 // One step of compact node own: pull, walls and faces, moments, collision, store.
-// HH, CURVED, EXT: whether the lattice may have wet-node walls, curved walls and
-// extrapolating 3D outlets (kernels for lattices without them leave the code out).
+// HH, CURVED, EXT as in post_boundary.
 template <class L, int S, int C, bool OPEN, bool HH = true, bool CURVED = true, bool EXT = true>
 __device__ inline void step_node(const typename Io<L, S>::raw* __restrict__ src,
                                  typename Io<L, S>::raw* __restrict__ dst, const uint32_t* __restrict__ didx,
@@ -69,46 +68,7 @@ __device__ inline void step_node(const typename Io<L, S>::raw* __restrict__ src,
     const int y = (int)(q1 - zq * (uint32_t)kp.ny), z = (int)zq;
     const uint32_t cls = nd >> kClsShift;
     T h[L::Q];
-    if constexpr (OPEN && L::Q == 19 && EXT) {
-        // An extrapolating outlet node takes its unknowns from the one or two
-        // nodes upstream: the pull, walls and faces of up to three nodes in a
-        // loop, so that their code is there once (three copies become calls,
-        // with the populations in scratch).
-        int nk = 1, dx = 0, dy = 0, dz = 0;
-        if (is_outlet3(cls) && (kp.outlet == 2 || kp.outlet == 3)) {
-            const int A = cls == PRES_E || cls == OUT_W ? 0 : (cls == OUT_S || cls == OUT_N ? 1 : 2);
-            const int G = cls == OUT_W || cls == OUT_S || cls == OUT_B ? 1 : -1;
-            dx = A == 0 ? G : 0; dy = A == 1 ? G : 0; dz = A == 2 ? G : 0;
-            const int n = kp.outlet == 2 ? 2 : 1;
-            const int ex = x + n * dx, ey = y + n * dy, ez = z + n * dz;
-            if (ex >= 0 && ex < kp.nx && ey >= 0 && ey < kp.ny && ez >= 0 && ez < kp.nz) nk = n + 1;
-        }
-        const int step = dx + (dy + dz * kp.ny) * kp.nx;
-        uint32_t oj[3] = {own, 0u, 0u};
-        if (nk > 1) {   // a solid node upstream: the streamed values stay
-            oj[1] = cidx[idx + (uint32_t)step];
-            oj[2] = nk > 2 ? cidx[idx + (uint32_t)(2 * step)] : 0u;
-            if (oj[1] == kNone || oj[2] == kNone) nk = 1;
-        }
-#pragma clang loop unroll(disable)
-        for (int k = 0; k < nk; ++k) {
-            const uint32_t j = k == 0 ? own : k == 1 ? oj[1] : oj[2];
-            T hk[L::Q];
-            inflow_state<L, S, OPEN, HH, CURVED>(src, kp, fl, cidx, j, nodew[j], x + k * dx, y + k * dy, z + k * dz,
-                                                 idx + (uint32_t)(k * step), hk);
-            extrap_term<L, T>(cls, k, kp.outlet == 2, hk, h);
-        }
-    } else {
-        inflow_state<L, S, OPEN, HH, CURVED>(src, kp, fl, cidx, own, nd, x, y, z, idx, h);
-    }
-    if (OPEN && L::Q == 9 && cls == PRES_E) {
-        zou_outlet<L, T>(kp, fl, idx, h);
-        outlet_extrap<L, S, OPEN>(src, kp, fl, cidx, nodew, true, x, y, z, idx, h);
-    }
-    if (OPEN && L::Q == 19) {
-        if (is_outlet3(cls) && kp.outlet != 2 && kp.outlet != 3) outlet3_local<L, S, OPEN>(kp, fl, idx, cls, h);
-        sym3d<L, T>(cls, h);
-    }
+    post_boundary<L, S, OPEN, false, HH, CURVED, EXT>(src, kp, fl, nodew, cidx, own, nd, x, y, z, idx, h);
     T drho, rho, u[3];
     moments<L, T>(kp, cls, h, drho, rho, u);
     if (OPEN) frozen_macros<T>(kp, fl, cls, idx, drho, rho, u);
