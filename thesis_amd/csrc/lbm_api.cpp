@@ -354,12 +354,13 @@ lbm_status lbm_create(const lbm_params* p, const lbm_lattice* lat, lbm_ctx** out
     // between, at 56 MiB of populations.
     std::vector<uint32_t> edge;
     const bool periodic3 = p->periodic[0] && p->periodic[1] && p->periodic[2];
-    if (p->q == 19 && !periodic3 && nf * 19 * storage_bytes(p->storage) >= (size_t)56 << 20) {
-        const bool ext = p->outlet_model == LBM_OUTLET_EXTRAP2 || p->outlet_model == LBM_OUTLET_EXTRAP1;
+    const bool ext = any_outlet && (p->outlet_model == LBM_OUTLET_EXTRAP2 || p->outlet_model == LBM_OUTLET_EXTRAP1);
+    const bool curved = p->wall_model == LBM_WALL_CURVED;
+    if (p->q == 19 && !periodic3 && (ext || curved) && nf * 19 * storage_bytes(p->storage) >= (size_t)56 << 20) {
         for (size_t j = 0; j < nf; ++j) {
             const uint32_t nd = nodew[j], cls = nd >> kClsShift;
             const bool outlet = ext && (cls == LBM_PRES_E || (cls >= LBM_OUT_W && cls <= LBM_OUT_T));
-            if (outlet || (p->wall_model == LBM_WALL_CURVED && (nd & kBBMask))) edge.push_back((uint32_t)j);
+            if (outlet || (curved && (nd & kBBMask))) edge.push_back((uint32_t)j);
         }
     }
     // Row metadata of the rank step: per row and 32-node word, the fluid mask
