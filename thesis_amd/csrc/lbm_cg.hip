@@ -242,7 +242,7 @@ __global__ __launch_bounds__(THREADS) void k_cg_step(const typename CIo<S>::raw*
 // with k_cg_step: there the conversion of a pulled value is fused into the density's
 // sum, and without that a rounding of 2^-11 falls the other way now and then.
 //
-// Per step, one launch a step / several (the number): FP64 64 x 64 7.3 / 3.6 us (6),
+// Per step, one launch a step / several (the number): FP64 64 x 64 7.3 / 3.5 us (7),
 // 250 x 187 8.1 / 4.5 (5), 512 x 512 17.6 / 15.2 (2), 1024 x 1024 69 / 52 (3); FP32
 // 5.8 / 2.8, 6.6 / 3.6, 10.3 / 8.4, 42 / 25; 24-point stencil FP64 250 x 187 8.5 / 5.5
 // (3), 1024 x 1024 76 / 66 (2).  What bounds it: on few squares the launch and the
